@@ -16,10 +16,11 @@
 //    small_pixels() pixel centres are rasterized right away (64-bit atomic min per covered
 //    pixel); the others are binned into 16x16 tiles. Per-tile counts gather in an LDS table of
 //    the workgroup before one global atomic per distinct tile.
-// 3. A three-phase scan turns tile counts into list offsets; the bin pass reserves each
-//    workgroup's share of a tile's list with one global atomic and fills it. Each tile has one
-//    list per depth slab (the triangle's nearest vertex within the image's depth span), so a
-//    tile's entries run near to far.
+//    Triangles over more than kLargeTiles tiles only join a list of large triangles.
+// 3. One pass turns the tile counts (and the large triangles over each tile) into places for
+//    the tile lists; the bin pass reserves each workgroup's share of a tile's list with one
+//    global atomic and fills it. Each tile has one list per depth slab (the triangle's nearest
+//    vertex within the image's depth span), so a tile's entries run near to far.
 // 4. One 256-thread workgroup per tile with entries (heavy tiles first, each XCD on its own
 //    share of the tiles) holds the tile's keys in LDS and walks its entries 256 at a time:
 //    triangles entirely behind the tile's farthest key are skipped; the others are staged in
@@ -52,15 +53,29 @@ static_assert(kWindow == 4 * 256, "the map scan gives each thread four entries")
 // with 16, 2.38 with 64).
 constexpr int kSmallPixelsDense = 8;
 constexpr int kSmallPixelsRanges = 64;
-constexpr int kScanBlock = 1024;     // elements per scan block (256 threads x 4)
+// Threads per workgroup of the list pass, with 4 lists each, or 1 where a tile has one list:
+// its workgroups all add to two counters, ~9 ns an addition (256 threads x 4: 35 us for 518 k
+// lists), but the large triangles over few tiles need workgroups to share them.
+constexpr int kListThreads = 1024;
 constexpr int kOrderBuckets = 4096;  // Morton buckets (12 bits of a 30-bit code)
 constexpr int kOrderMinTris = 8192;  // smaller meshes keep their own order
 constexpr int kTileSlots = 1024;     // LDS table of a workgroup's tiles
 constexpr int kRecord = 4;           // float4 per binned triangle record (one 64-byte line)
 constexpr int kDepthSlabs = 16;      // tile lists per tile, by the triangle's nearest depth
                                      // (dense views; range mode keeps one list per tile)
+constexpr int64_t kSlabsFrom = 8;    // triangles per tile from which instanced meshes use them
 constexpr int kRangeParts = 64;      // workgroups per image in the depth span reduction
 constexpr int kXcdShares = 8;        // XCDs of an MI355X: workgroup b runs on XCD b mod 8
+constexpr int kCounters = 5;
+// A triangle over more tiles than this is binned by the workgroups that own the tiles, not by
+// its own thread, which walks its tiles one after another (two table steps per tile).
+// Dense meshes, whose many workgroups hide that walk, keep it up to kLargeTilesDense tiles:
+// every list workgroup reads every large triangle. Rasterize calls, this limit 8 against 64:
+// 224 triangles at 2160 x 3840 329 / 372 us, 512 at 1448^2 103 / 1452 us, 4096 at 2 x 2048^2
+// 350 / 1164 us; 1.31 M noisy ones at 8 x 1024^2: list and bin passes 348 / 184 us.
+constexpr uint32_t kLargeTiles = 8;
+constexpr uint32_t kLargeTilesDense = 64;
+constexpr int64_t kLargeDenseFrom = (int64_t)1 << 18;  // triangle instances
 
 struct Workspace {
   float4* records;           // binned triangles, kRecord float4 each: the three clip-space
@@ -74,15 +89,16 @@ struct Workspace {
   // nearest depth falls in depth slab `slab` of their image, so a tile's entries are one range
   // that runs near to far.
   uint32_t* list_counts;     // [lists + 1]
-  uint32_t* list_offsets;    // [lists + 1] exclusive prefix of list_counts
-  uint32_t* list_cursor;     // [lists + 1] fill positions of the bin pass
-  uint32_t* chunk_offsets;   // [lists + 1] exclusive prefix of ceil(count / kChunk)
+  uint32_t* list_offsets;    // [lists + 1] where each list starts among the entries
+  uint32_t* list_cursor;     // [lists + 1] fill positions of the bin pass (then the lists' ends)
+  uint32_t* large;           // [lists + 1] records of the large triangles (counters[4] of them)
   uint32_t* depth_range;     // [depth_ranges][2] order-preserving bits of the nearest and
                              // farthest vertex depth of an image (one when pos is shared)
   uint32_t* range_parts;     // [depth_ranges][kRangeParts][2] partial spans
-  uint2* block_sums;         // [scan blocks] (entries, chunks)
   uint32_t* counters;        // [0] setup workgroups, [1] entries, [2] tile pass
-                             // workgroups, [3] busy tiles
+                             // workgroups, [3] busy tiles, [4] large triangles (those beyond
+                             // the list's capacity went the ordinary way)
+  uint32_t* lists_done;      // workgroups of the list pass that are done
   uint32_t* block_records;   // [record_blocks] binned triangles of each setup workgroup
   uint32_t* tile_order;      // [tiles] tile pass order: heavy tiles first within each XCD's share
   uint8_t* tile_class;       // [tiles] work class of each tile (entries / 32, capped)
@@ -103,9 +119,10 @@ struct Workspace {
   int64_t tiles;
   int64_t lists;
   int depth_ranges;
-  int scan_blocks;
+  int list_blocks;
   int record_blocks;          // setup workgroups; each owns 256 record slots
   int slabs;                  // tile lists per tile: kDepthSlabs, or 1 in range mode
+  uint32_t large_limit;       // a triangle over more tiles than this is a large one
   size_t bytes;
 };
 
@@ -113,6 +130,10 @@ size_t align_up(size_t v) { return (v + 255) & ~size_t(255); }
 
 int small_pixels(const DrRasterGeometry& g) {
   return g.ranges != nullptr ? kSmallPixelsRanges : kSmallPixelsDense;
+}
+
+uint32_t large_tiles_limit(const DrRasterGeometry& g) {
+  return g.num_instances < kLargeDenseFrom ? kLargeTiles : kLargeTilesDense;
 }
 
 bool use_order(const DrRasterGeometry& g) {
@@ -127,9 +148,15 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
   // Range mode keeps one list per tile: its items' triangles mostly take the small-triangle path,
   // so the near-to-far slabs gain its tile pass nothing, while their lists (clears, scans) and
   // the depth span they need cost 0.2 ms per step of four layers of 256 items at 512 x 512.
-  w.slabs = g.ranges != nullptr ? 1 : kDepthSlabs;
+  // So do meshes of few triangles per tile, whose lists fit one chunk of the tile pass in most
+  // tiles: the slabs order chunks (20 k triangles at 8 x 1024^2, 5 per tile: rasterize 283 us
+  // with slabs, 259 without; at 20 per tile 474 and 495).
+  w.slabs = g.ranges != nullptr || g.num_tri <= kSlabsFrom * w.tiles_x * w.tiles_y ? 1
+                                                                                  : kDepthSlabs;
   w.lists = w.tiles * w.slabs;
-  w.scan_blocks = (int)((w.lists + 1 + kScanBlock - 1) / kScanBlock);
+  w.large_limit = large_tiles_limit(g);
+  const int64_t list_block = (int64_t)kListThreads * (w.slabs == 1 ? 1 : 4);
+  w.list_blocks = (int)((w.lists + list_block - 1) / list_block);
   w.depth_ranges = (g.ranges == nullptr && g.pos_batch_stride != 0) ? std::max(g.batch, 1) : 1;
   w.ordered = use_order(g);
   w.record_blocks = std::max(blocks_for(g.num_instances, 256), 1);
@@ -139,14 +166,14 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
     off = align_up(off + bytes);
     return p;
   };
-  w.counters = (uint32_t*)take(16);
+  w.counters = (uint32_t*)take(kCounters * sizeof(uint32_t));
+  w.lists_done = (uint32_t*)take(sizeof(uint32_t));
   w.list_counts = (uint32_t*)take(sizeof(uint32_t) * (w.lists + 1));
   w.list_offsets = (uint32_t*)take(sizeof(uint32_t) * (w.lists + 1));
   w.list_cursor = (uint32_t*)take(sizeof(uint32_t) * (w.lists + 1));
-  w.chunk_offsets = (uint32_t*)take(sizeof(uint32_t) * (w.lists + 1));
+  w.large = (uint32_t*)take(sizeof(uint32_t) * (w.lists + 1));
   w.depth_range = (uint32_t*)take(sizeof(uint32_t) * 2 * w.depth_ranges);
   w.range_parts = (uint32_t*)take(sizeof(uint32_t) * 2 * kRangeParts * w.depth_ranges);
-  w.block_sums = (uint2*)take(sizeof(uint2) * (w.scan_blocks + 1));
   w.block_records = (uint32_t*)take(sizeof(uint32_t) * w.record_blocks);
   w.tile_order = (uint32_t*)take(sizeof(uint32_t) * w.tiles);
   w.tile_class = (uint8_t*)take(w.tiles);
@@ -335,6 +362,11 @@ __device__ __forceinline__ void merge_key(uint64_t* keys, const uint64_t* prev, 
   atomicMin((unsigned long long*)(keys + pixel), (unsigned long long)key);
 }
 
+// Room in the list of large triangles.
+__device__ __forceinline__ uint32_t large_capacity(const Workspace& ws) {
+  return (uint32_t)(ws.lists + 1);
+}
+
 // ---- workgroup table of tiles -------------------------------------------------------------
 
 // Counts (and, in the bin pass, list reservations) per distinct tile of a workgroup, in LDS.
@@ -393,7 +425,8 @@ __global__ void raster_prepare(uint64_t* keys, int64_t pixels, Workspace ws, int
   for (int64_t i = t; i < kXcdShares * kWorkClasses; i += stride) ws.class_counts[i] = 0u;
   if (ws.ordered)
     for (int64_t i = t; i < kOrderBuckets; i += stride) ws.bucket_counts[i] = 0u;
-  if (t < 4) ws.counters[t] = t == 0 ? (uint32_t)ws.record_blocks : 0u;
+  if (t < kCounters) ws.counters[t] = t == 0 ? (uint32_t)ws.record_blocks : 0u;
+  if (t == 0) *ws.lists_done = 0u;
   for (int64_t i = t; i < width; i += stride) ws.px[i] = pixel_centre((int)i, width);
   for (int64_t i = t; i < height; i += stride) ws.py[i] = pixel_centre((int)i, height);
 }
@@ -871,22 +904,40 @@ __global__ __launch_bounds__(256) void raster_setup_kernel(DrRasterGeometry g,
       float4* out = ws.records + (size_t)rec * kRecord;
 #pragma unroll
       for (int k = 0; k < 3; ++k) out[k] = make_float4(T.x[k], T.y[k], T.z[k], T.w[k]);
-      const uint32_t tx_range = (uint32_t)tx0 | ((uint32_t)tx1 << 16);
-      const uint32_t ty_range = (uint32_t)ty0 | ((uint32_t)ty1 << 16);
+      // A large triangle joins the list of large triangles while there is room (one counter
+      // update per wave).
+      bool large = (uint32_t)(tx1 - tx0 + 1) * (uint32_t)(ty1 - ty0 + 1) > ws.large_limit;
+      const uint64_t larges = __ballot(large);
+      if (larges != 0) {
+        const int leader = __ffsll((unsigned long long)larges) - 1;
+        uint32_t first = 0u;
+        if (lane == leader) first = atomicAdd(ws.counters + 4, (uint32_t)__popcll(larges));
+        first = (uint32_t)__shfl((int)first, leader) +
+                (uint32_t)__popcll(larges & ((1ull << lane) - 1ull));
+        large = large && first < large_capacity(ws);
+        if (large) ws.large[first] = rec;
+      }
+      // Its tile range is kept with the ends swapped: an empty range to the bin pass, which
+      // leaves it to the tiles' workgroups (large_tiles).
+      const uint32_t tx_range = large ? (uint32_t)tx1 | ((uint32_t)tx0 << 16)
+                                      : (uint32_t)tx0 | ((uint32_t)tx1 << 16);
+      const uint32_t ty_range = large ? (uint32_t)ty1 | ((uint32_t)ty0 << 16)
+                                      : (uint32_t)ty0 | ((uint32_t)ty1 << 16);
       out[3] = make_float4(__int_as_float(b), __int_as_float(t | (slab << 24)),
                            __uint_as_float(tx_range), __uint_as_float(ty_range));
       const uint32_t list0 = (uint32_t)b * ws.tiles_x * ws.tiles_y * ws.slabs + (uint32_t)slab;
       ws.record_bins[rec] =
           make_uint4(tx_range, ty_range, list0, __float_as_uint(depth_lower_bound(T)));
-      for (int ty = ty0; ty <= ty1; ++ty)
-        for (int tx = tx0; tx <= tx1; ++tx) {
-          const uint32_t list = list0 + (uint32_t)(ty * ws.tiles_x + tx) * ws.slabs;
-          const int slot = table.insert(list);
-          if (slot >= 0)
-            atomicAdd(table.count + slot, 1u);
-          else
-            atomicAdd(ws.list_counts + list, 1u);
-        }
+      if (!large)
+        for (int ty = ty0; ty <= ty1; ++ty)
+          for (int tx = tx0; tx <= tx1; ++tx) {
+            const uint32_t list = list0 + (uint32_t)(ty * ws.tiles_x + tx) * ws.slabs;
+            const int slot = table.insert(list);
+            if (slot >= 0)
+              atomicAdd(table.count + slot, 1u);
+            else
+              atomicAdd(ws.list_counts + list, 1u);
+          }
     }
   }
   __syncthreads();
@@ -894,98 +945,262 @@ __global__ __launch_bounds__(256) void raster_setup_kernel(DrRasterGeometry g,
     if (table.key[s] != TileTable::kEmpty) atomicAdd(ws.list_counts + table.key[s], table.count[s]);
 }
 
-// Inclusive scan of (entries, chunks) pairs over the 256 threads of a block.
-__device__ __forceinline__ uint2 block_inclusive_scan(uint2 v, uint2* lds) {
-  const int lane = lane_id();
-  const int wave = threadIdx.x / DR_WAVE;
+// ---- kernels: tile lists ------------------------------------------------------------------
+//
+// The lists' places among the entries, and the tile pass's order: heavy tiles first within each
+// XCD's share. The tile pass takes the busy tiles in their XCD shares' order (so that XCD k,
+// which takes the k-th eighth of the workgroups under xcd_order, gets about share k), within a
+// share the tiles with the most binned triangles first, so that the longest workgroups do not
+// start last: a counting sort by entry count in kWorkClasses classes of 32 entries. The order
+// within a class is free: tiles are independent.
+
+// The XCD share of tile i under xcd_order, and the first tile of share k.
+__device__ __forceinline__ int xcd_share(int64_t i, int64_t tiles) {
+  if (tiles < kXcdShares) return (int)i;
+  const int64_t per = tiles / kXcdShares, extra = tiles % kXcdShares;
+  const int64_t big = extra * (per + 1);
+  return i < big ? (int)(i / (per + 1)) : (int)(extra + (i - big) / per);
+}
+
+// Calls f(list - first_list, record, depth bound bits) for every tile list of
+// [first_list, first_list + lists) that a large triangle belongs to. Each lane looks at a large
+// triangle of its own; those that share tiles with the workgroup's are then walked by the whole
+// wave, 64 tiles of the shared rows at once. Large triangles are few next to the tiles they
+// cover, and a workgroup passes over all of them in a fraction of the time one thread would
+// walk one's tiles. Whole waves call this.
+template <typename F>
+__device__ __forceinline__ void large_tiles(const Workspace& ws, int64_t first_list, int lists,
+                                            uint32_t count, F f) {
+  const int64_t first_tile = first_list / ws.slabs;
+  const int64_t past_tile = min((first_list + lists) / ws.slabs, ws.tiles);
+  const int64_t per_image = (int64_t)ws.tiles_x * ws.tiles_y;
+  const uint32_t lane = lane_id();
+  for (uint32_t i0 = threadIdx.x - lane; i0 < count; i0 += blockDim.x) {  // uniform
+    const uint32_t rec = ws.large[min(i0 + lane, count - 1)];
+    const uint4 info = ws.record_bins[rec];
+    const int tx0 = (int)(info.x >> 16), tx1 = (int)(info.x & 0xffffu);  // stored swapped
+    const int ty0 = (int)(info.y >> 16), ty1 = (int)(info.y & 0xffffu);
+    const int64_t image_tile = info.z / (uint32_t)ws.slabs;  // the image's first tile
+    // The workgroup's tiles [from, to) relative to the image's, and its rows among them.
+    const int from = (int)min(max(first_tile - image_tile, (int64_t)0), per_image);
+    const int to = (int)min(max(past_tile - image_tile, (int64_t)0), per_image);
+    const int row0 = max(ty0, from / ws.tiles_x);
+    const int row1 = min(ty1, (to - 1) / ws.tiles_x);
+    uint64_t hits = __ballot(i0 + lane < count && from < to && row0 <= row1);
+    while (hits != 0) {
+      const int j = __ffsll((unsigned long long)hits) - 1;
+      hits &= hits - 1;
+      const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)rec, j);
+      const uint32_t bits = (uint32_t)__builtin_amdgcn_readlane((int)info.w, j);
+      const uint32_t list0 = (uint32_t)__builtin_amdgcn_readlane((int)info.z, j);
+      const int x0 = __builtin_amdgcn_readlane(tx0, j), x1 = __builtin_amdgcn_readlane(tx1, j);
+      const int y0 = __builtin_amdgcn_readlane(row0, j), y1 = __builtin_amdgcn_readlane(row1, j);
+      const int lo = __builtin_amdgcn_readlane(from, j), hi = __builtin_amdgcn_readlane(to, j);
+      // List 0 of the image's tile 0 in the triangle's slab, from the workgroup's first list.
+      const int64_t origin = (int64_t)list0 - first_list;
+      const uint32_t wide = (uint32_t)(x1 - x0 + 1), cells = wide * (uint32_t)(y1 - y0 + 1);
+      for (uint32_t p = lane; p < cells; p += DR_WAVE) {
+        const uint32_t dy = p / wide;
+        const int tile = (y0 + (int)dy) * ws.tiles_x + x0 + (int)(p - dy * wide);
+        if (tile >= lo && tile < hi) f((int)(origin + (int64_t)tile * ws.slabs), r, bits);
+      }
+    }
+  }
+}
+
+// One workgroup per PER lists a thread (whole tiles: one list each with PER = 1, else four
+// threads' lists): the large triangles over each list are counted in LDS, a scan over the workgroup's lists and one
+// addition to the entry count give every list its place -- a tile's lists in one range, near to
+// far; where the workgroup's ranges lie among the others' does not matter -- and each tile's
+// work class joins the class counts of its XCD share. The last workgroup to finish turns those
+// into the classes' first positions. (A three-phase scan of the lists, a pass for the classes
+// and one for the cursors before: five launches of 2-5 us each; one now.)
+template <int PER>
+__global__ __launch_bounds__(kListThreads) void raster_list_kernel(Workspace ws) {
+  constexpr int kListBlock = PER * kListThreads;
+  __shared__ uint32_t s_large[kListBlock];
+  __shared__ uint32_t s_hist[kXcdShares * kWorkClasses];
+  __shared__ uint32_t s_wave[kListThreads / DR_WAVE];
+  __shared__ uint32_t s_first;
+  __shared__ bool s_last;
+  static_assert(PER == 1 || 4 * PER == kDepthSlabs, "a thread or four of them per tile");
+  static_assert(kXcdShares * kWorkClasses == kListThreads, "a class per thread");
+  const int lane = lane_id(), wave = threadIdx.x / DR_WAVE;
+  const int64_t first_list = (int64_t)blockIdx.x * kListBlock;
+  const int64_t i0 = first_list + PER * threadIdx.x;
+  uint32_t count[PER];
 #pragma unroll
-  for (int d = 1; d < DR_WAVE; d <<= 1) {
-    uint32_t ax = __shfl_up(v.x, d), ay = __shfl_up(v.y, d);
-    if (lane >= d) {
-      v.x += ax;
-      v.y += ay;
-    }
-  }
-  if (lane == DR_WAVE - 1) lds[wave] = v;
+  for (int k = 0; k < PER; ++k) count[k] = i0 + k < ws.lists ? ws.list_counts[i0 + k] : 0u;
+  const uint32_t larges = min(ws.counters[4], large_capacity(ws));  // uniform over the grid
+#pragma unroll
+  for (int k = 0; k < PER; ++k) s_large[PER * threadIdx.x + k] = 0u;
+  s_hist[threadIdx.x] = 0u;
   __syncthreads();
-  uint2 offset = make_uint2(0, 0);
-  for (int k = 0; k < wave; ++k) {
-    offset.x += lds[k].x;
-    offset.y += lds[k].y;
-  }
-  __syncthreads();
-  return make_uint2(v.x + offset.x, v.y + offset.y);
-}
-
-__device__ __forceinline__ uint2 scan_item(const uint32_t* counts, int64_t i, int64_t n) {
-  uint32_t c = i < n ? counts[i] : 0u;
-  return make_uint2(c, (c + kChunk - 1) / kChunk);
-}
-
-// Phase 1: per-block totals.
-__global__ __launch_bounds__(256) void raster_scan_reduce(const uint32_t* counts, int64_t n,
-                                                          uint2* block_sums) {
-  __shared__ uint2 lds[4];
-  const int64_t base = (int64_t)blockIdx.x * kScanBlock + threadIdx.x * 4;
-  uint2 s = make_uint2(0, 0);
-  for (int k = 0; k < 4; ++k) {
-    uint2 v = scan_item(counts, base + k, n);
-    s.x += v.x;
-    s.y += v.y;
-  }
-  uint2 total = block_inclusive_scan(s, lds);
-  if (threadIdx.x == 255) block_sums[blockIdx.x] = total;
-}
-
-// Phase 2: exclusive scan of the block totals in one block; totals go to the counters.
-__global__ __launch_bounds__(256) void raster_scan_blocks(uint2* block_sums, int blocks,
-                                                          uint32_t* counters) {
-  __shared__ uint2 lds[4];
-  __shared__ uint2 step_total;
-  uint2 carry = make_uint2(0, 0);
-  for (int start = 0; start < blocks; start += 256) {
-    const int i = start + threadIdx.x;
-    const uint2 v = i < blocks ? block_sums[i] : make_uint2(0, 0);
-    const uint2 inc = block_inclusive_scan(v, lds);
-    if (i < blocks) block_sums[i] = make_uint2(carry.x + inc.x - v.x, carry.y + inc.y - v.y);
-    if (threadIdx.x == 255) step_total = inc;
-    __syncthreads();
-    carry.x += step_total.x;
-    carry.y += step_total.y;
+  if (larges != 0) {
+    large_tiles(ws, first_list, kListBlock, larges,
+                [&](int list, uint32_t, uint32_t) { atomicAdd(s_large + list, 1u); });
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    counters[1] = carry.x;
+  uint32_t large[PER], total[PER], sum = 0u;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    large[k] = s_large[PER * threadIdx.x + k];
+    total[k] = count[k] + large[k];
+    sum += total[k];
+  }
+  const uint32_t incl = wave_inclusive_sum(sum);
+  if (lane == DR_WAVE - 1) s_wave[wave] = incl;
+  // Each tile's class: none, then one per 32 entries, the last one open-ended. A tile is four
+  // lists of each of four lanes, or one list.
+  auto classify = [&](int64_t tile, uint32_t n) {
+    if (tile >= ws.tiles) return;
+    const int c = n == 0 ? 0 : (int)min((n >> 5) + 1, (uint32_t)(kWorkClasses - 1));
+    ws.tile_class[tile] = (uint8_t)c;
+    atomicAdd(s_hist + xcd_share(tile, ws.tiles) * kWorkClasses + c, 1u);
+  };
+  if constexpr (PER == 1) {
+    classify(i0, total[0]);
+  } else {
+    uint32_t n = sum + (uint32_t)__shfl_xor((int)sum, 1);
+    n += (uint32_t)__shfl_xor((int)n, 2);
+    if ((lane & 3) == 0) classify(i0 / kDepthSlabs, n);
+  }
+  __syncthreads();
+  uint32_t before = 0u, all = 0u;
+#pragma unroll
+  for (int w = 0; w < kListThreads / DR_WAVE; ++w) {
+    before += w < wave ? s_wave[w] : 0u;
+    all += s_wave[w];
+  }
+  if (threadIdx.x == 0) s_first = all != 0u ? atomicAdd(ws.counters + 1, all) : 0u;
+  const uint32_t in_class = s_hist[threadIdx.x];
+  if (in_class != 0u) atomicAdd(ws.class_counts + threadIdx.x, in_class);
+  // The class counts change through device atomics alone, which are performed beyond the L2s:
+  // once every thread's are acknowledged, the last workgroup's reads past its L2 find them all.
+  // (A device-scope release would also write this XCD's L2 back: 20 us instead of 10 for
+  // 524 k lists.)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  uint32_t at = s_first + before + incl - sum;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if (i0 + k < ws.lists) {
+      ws.list_offsets[i0 + k] = at;
+      ws.list_cursor[i0 + k] = at + large[k];  // the large triangles' entries come first
+    }
+    at += total[k];
+  }
+  // After the barrier above: every class count of the workgroup is in place.
+  if (threadIdx.x == 0) s_last = atomicAdd(ws.lists_done, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!s_last) return;  // uniform over the workgroup
+
+  // The first position of each class: the busy tiles share by share, heaviest class first
+  // within a share, then the tiles without entries. Thread t takes share k = t / 32 and its
+  // classes 127 - 4s .. 124 - 4s (s = t % 32), heaviest first; class 0 is counted apart. (The
+  // counts come from other workgroups of this launch: read past this XCD's L2.)
+  static_assert(kXcdShares * 32 == 256 && kWorkClasses == 4 * 32,
+                "32 threads per share, 4 classes each");
+  __shared__ uint32_t busy[kXcdShares], idle[kXcdShares];
+  auto class_count = [&](int i) {
+    return __hip_atomic_load(ws.class_counts + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const int k = threadIdx.x / 32, s = threadIdx.x % 32;  // threads past 256: no share
+  uint32_t v[4], local = 0u;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = kWorkClasses - 1 - 4 * s - q;
+    v[q] = c >= 1 && k < kXcdShares ? class_count(k * kWorkClasses + c) : 0u;
+    local += v[q];
+  }
+  // Exclusive prefix of the share's classes in that order: a wave holds two shares (lanes 0-31
+  // and 32-63), so the upper half drops the lower half's total.
+  const uint32_t class_incl = wave_inclusive_sum(local);
+  const uint32_t lower = (uint32_t)__builtin_amdgcn_readlane((int)class_incl, 31);
+  const uint32_t share_incl = lane >= 32 ? class_incl - lower : class_incl;
+  if (s == 31 && k < kXcdShares) {
+    busy[k] = share_incl;
+    idle[k] = class_count(k * kWorkClasses);
+  }
+  __syncthreads();
+  if (k >= kXcdShares) return;
+  uint32_t first = 0u, idle_first = 0u, widest = 0u;
+#pragma unroll
+  for (int j = 0; j < kXcdShares; ++j) {
+    first += j < k ? busy[j] : 0u;
+    idle_first += busy[j] + (j < k ? idle[j] : 0u);
+    widest = max(widest, busy[j]);
+  }
+  uint32_t place = first + share_incl - local;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = kWorkClasses - 1 - 4 * s - q;
+    if (c >= 1) ws.class_cursor[k * kWorkClasses + c] = place;
+    place += v[q];
+  }
+  if (s == 0) {
+    ws.class_cursor[k * kWorkClasses] = idle_first;
+    ws.share_info[k] = busy[k];
+    ws.share_info[kXcdShares + k] = first;
+    if (k == 0) {
+      ws.counters[2] = kXcdShares * widest;  // the tile pass's workgroups
+      ws.counters[3] = idle_first;           // the busy tiles
+    }
   }
 }
 
-// Phase 3: exclusive offsets per tile (and the totals at index n).
-__global__ __launch_bounds__(256) void raster_scan_apply(const uint32_t* counts, int64_t n,
-                                                         const uint2* block_sums,
-                                                         uint32_t* offsets, uint32_t* cursor,
-                                                         uint32_t* chunk_offsets) {
-  __shared__ uint2 lds[4];
-  const int64_t base = (int64_t)blockIdx.x * kScanBlock + threadIdx.x * 4;
-  uint2 items[4];
-  uint2 s = make_uint2(0, 0);
-  for (int k = 0; k < 4; ++k) {
-    items[k] = scan_item(counts, base + k, n);
-    s.x += items[k].x;
-    s.y += items[k].y;
+// ---- kernels: bin -------------------------------------------------------------------------
+
+// What 256 tiles need besides the records' entries: their places in the tile pass's order
+// (positions reserved per class) and the large triangles' entries.
+struct TileStage {
+  uint32_t hist[kXcdShares * kWorkClasses];
+  uint32_t base[kXcdShares * kWorkClasses];
+};
+constexpr int kStageTiles = 256;
+
+__device__ __forceinline__ void place_tiles(const Workspace& ws, TileStage& p, int block) {
+  for (int i = threadIdx.x; i < kXcdShares * kWorkClasses; i += blockDim.x) p.hist[i] = 0u;
+  __syncthreads();
+  const int64_t tile = (int64_t)block * kStageTiles + threadIdx.x;
+  int slot = 0;
+  if (tile < ws.tiles) {
+    slot = xcd_share(tile, ws.tiles) * kWorkClasses + ws.tile_class[tile];
+    atomicAdd(p.hist + slot, 1u);
   }
-  uint2 inc = block_inclusive_scan(s, lds);
-  uint2 run = make_uint2(block_sums[blockIdx.x].x + inc.x - s.x,
-                         block_sums[blockIdx.x].y + inc.y - s.y);
-  for (int k = 0; k < 4; ++k) {
-    const int64_t i = base + k;
-    if (i <= n) {
-      offsets[i] = run.x;
-      chunk_offsets[i] = run.y;
-      if (i < n) cursor[i] = run.x;
-    }
-    run.x += items[k].x;
-    run.y += items[k].y;
+  __syncthreads();
+  constexpr int kClassesPerThread = kXcdShares * kWorkClasses / 256;
+  uint32_t reserved[kClassesPerThread];
+#pragma unroll
+  for (int k = 0; k < kClassesPerThread; ++k) {
+    const int i = threadIdx.x + k * 256;
+    reserved[k] = p.hist[i] ? atomicAdd(ws.class_cursor + i, p.hist[i]) : 0u;
   }
+#pragma unroll
+  for (int k = 0; k < kClassesPerThread; ++k) {
+    const int i = threadIdx.x + k * 256;
+    p.base[i] = reserved[k];
+    p.hist[i] = 0u;
+  }
+  __syncthreads();
+  if (tile < ws.tiles) ws.tile_order[p.base[slot] + atomicAdd(p.hist + slot, 1u)] = (uint32_t)tile;
+}
+
+// The large triangles' entries, at the front of each list (raster_list_kernel left room for
+// exactly these).
+__device__ __forceinline__ void bin_large(const Workspace& ws,
+                                          uint32_t (&filled)[kStageTiles * kDepthSlabs],
+                                          uint2* entries, int block) {
+  const uint32_t larges = min(ws.counters[4], large_capacity(ws));
+  if (larges == 0) return;  // uniform over the grid
+  const int lists = kStageTiles * ws.slabs;
+  for (int i = threadIdx.x; i < lists; i += blockDim.x) filled[i] = 0u;
+  __syncthreads();
+  const int64_t first_list = (int64_t)block * lists;
+  large_tiles(ws, first_list, lists, larges, [&](int list, uint32_t rec, uint32_t bound_bits) {
+    entries[ws.list_offsets[first_list + list] + atomicAdd(filled + list, 1u)] =
+        make_uint2(rec, bound_bits);
+  });
 }
 
 // Fills the per-tile lists: the workgroup counts its records per tile in LDS, reserves its
@@ -995,22 +1210,19 @@ __global__ __launch_bounds__(256) void raster_scan_apply(const uint32_t* counts,
 // (bin pass 186 -> 163 us at 8 x 1024^2 with two; 172 us with four).
 constexpr int kBinBlocks = 2;
 
-__global__ __launch_bounds__(256) void raster_bin_kernel(Workspace ws, uint2* entries,
-                                                         uint32_t capacity) {
-  // Entries beyond the buffer's capacity: the pass is left to a later launch with a larger
-  // buffer (the cursors stay untouched, so that launch places every entry).
-  if (ws.counters[1] > capacity) return;  // uniform over the grid
-  __shared__ TileTable table;
+__device__ __forceinline__ void bin_records(const Workspace& ws, TileTable& table,
+                                            uint2* entries, int bin_block) {
   table.clear();
   __syncthreads();
   // This thread's record of each of the workgroup's setup workgroups: tile range, first list,
   // and the triangle's depth bound, which each entry carries so that the tile pass can skip a
-  // triangle behind every key of its tile without reading its record.
+  // triangle behind every key of its tile without reading its record. (Large triangles' ranges
+  // are stored swapped: empty.)
   int tx0[kBinBlocks], tx1[kBinBlocks], ty0[kBinBlocks], ty1[kBinBlocks];
   uint32_t list0[kBinBlocks], bound_bits[kBinBlocks], rec[kBinBlocks];
 #pragma unroll
   for (int q = 0; q < kBinBlocks; ++q) {
-    const int block = (int)blockIdx.x * kBinBlocks + q;
+    const int block = bin_block * kBinBlocks + q;
     tx0[q] = ty0[q] = 0;
     tx1[q] = ty1[q] = -1;
     list0[q] = bound_bits[q] = 0u;
@@ -1062,138 +1274,34 @@ __global__ __launch_bounds__(256) void raster_bin_kernel(Workspace ws, uint2* en
       }
 }
 
-static int bin_grid(const Workspace& ws) {
-  return (ws.record_blocks + kBinBlocks - 1) / kBinBlocks;
-}
-
-// ---- tile order: heavy tiles first within each XCD's share -----------------------------------
-//
-// The tile pass takes tiles in this order: the busy tiles in their XCD shares' order (so that
-// XCD k, which takes the k-th eighth of the workgroups under xcd_order, gets about share k),
-// within a share the tiles with the most binned triangles first, so that the longest
-// workgroups do not start last. A counting sort by entry count in kWorkClasses
-// classes of 32 entries, in three passes over the tiles (classes and their counts, the class
-// cursors, placement); workgroups aggregate in LDS before touching global counters. The order
-// within a class is free: tiles are independent.
-
-// The XCD share of tile i under xcd_order, and the first tile of share k.
-__device__ __forceinline__ int xcd_share(int64_t i, int64_t tiles) {
-  if (tiles < kXcdShares) return (int)i;
-  const int64_t per = tiles / kXcdShares, extra = tiles % kXcdShares;
-  const int64_t big = extra * (per + 1);
-  return i < big ? (int)(i / (per + 1)) : (int)(extra + (i - big) / per);
-}
-__device__ __forceinline__ int64_t share_start(int k, int64_t tiles) {
-  if (tiles < kXcdShares) return k;
-  const int64_t per = tiles / kXcdShares, extra = tiles % kXcdShares;
-  return k * per + (k < extra ? k : extra);
-}
-
-// Pass 1, one thread per tile: its class (kept for pass 3), the class counts of each share and
-// the number of tiles with binned triangles (counters[3], the tile pass's busy workgroups).
-__global__ __launch_bounds__(256) void raster_tile_classes(Workspace ws) {
-  __shared__ uint32_t hist[kXcdShares * kWorkClasses];
-  __shared__ uint32_t busy;
-  for (int i = threadIdx.x; i < kXcdShares * kWorkClasses; i += blockDim.x) hist[i] = 0u;
-  if (threadIdx.x == 0) busy = 0u;
-  __syncthreads();
-  const int64_t tile = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  bool has = false;
-  if (tile < ws.tiles) {
-    const uint32_t n =
-        ws.list_offsets[(tile + 1) * ws.slabs] - ws.list_offsets[tile * ws.slabs];
-    // Class 0: no entries; then one class per 32 entries, the last one open-ended.
-    const int c = n == 0 ? 0 : (int)min((n >> 5) + 1, (uint32_t)(kWorkClasses - 1));
-    ws.tile_class[tile] = (uint8_t)c;
-    atomicAdd(hist + xcd_share(tile, ws.tiles) * kWorkClasses + c, 1u);
-    has = n > 0;
-  }
-  const uint64_t mask = __ballot(has);
-  if (lane_id() == 0 && mask != 0) atomicAdd(&busy, (uint32_t)__popcll(mask));
-  __syncthreads();
-  for (int i = threadIdx.x; i < kXcdShares * kWorkClasses; i += blockDim.x)
-    if (hist[i]) atomicAdd(ws.class_counts + i, hist[i]);
-  if (threadIdx.x == 0 && busy) atomicAdd(ws.counters + 3, busy);
-}
-
-// Pass 2, one workgroup: first position of each class. The busy tiles come first, share by
-// share, heaviest class first within a share; the tiles without entries follow, so that the
-// tile pass launches one workgroup per busy tile. The classes' offsets are a scan over 32
-// threads per share (a serial walk over the 128 classes, writing each cursor twice, took 10 us).
-__global__ __launch_bounds__(256) void raster_tile_cursors(Workspace ws) {
-  static_assert(kXcdShares * 32 == 256 && kWorkClasses == 4 * 32,
-                "32 threads per share, 4 classes each");
-  __shared__ uint32_t busy[kXcdShares], idle[kXcdShares];
-  // Thread t takes share k = t / 32 and its classes 127 - 4s .. 124 - 4s (s = t % 32), heaviest
-  // first; class 0 (no entries) is counted apart.
-  const int k = threadIdx.x / 32, s = threadIdx.x % 32;
-  uint32_t v[4], local = 0u;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int c = kWorkClasses - 1 - 4 * s - q;
-    v[q] = c >= 1 ? ws.class_counts[k * kWorkClasses + c] : 0u;
-    local += v[q];
-  }
-  // Exclusive prefix of the share's classes in that order: a wave holds two shares (lanes 0-31
-  // and 32-63), so the upper half drops the lower half's total.
-  const uint32_t incl = wave_inclusive_sum(local);
-  const uint32_t lower = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
-  const uint32_t share_incl = lane_id() >= 32 ? incl - lower : incl;
-  if (s == 31) {
-    busy[k] = share_incl;
-    idle[k] = ws.class_counts[k * kWorkClasses];
-  }
-  __syncthreads();
-  uint32_t first = 0u, idle_first = 0u, widest = 0u;
-#pragma unroll
-  for (int j = 0; j < kXcdShares; ++j) {
-    first += j < k ? busy[j] : 0u;
-    idle_first += busy[j] + (j < k ? idle[j] : 0u);
-    widest = max(widest, busy[j]);
-  }
-  uint32_t at = first + share_incl - local;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int c = kWorkClasses - 1 - 4 * s - q;
-    if (c >= 1) ws.class_cursor[k * kWorkClasses + c] = at;
-    at += v[q];
-  }
-  if (s == 0) {
-    ws.class_cursor[k * kWorkClasses] = idle_first;
-    ws.share_info[k] = busy[k];
-    ws.share_info[kXcdShares + k] = first;
-    if (k == 0) ws.counters[2] = kXcdShares * widest;  // the tile pass's workgroups
+// The bin pass: the first `tile_blocks` workgroups place 256 tiles each in the tile pass's order
+// and bin their large triangles, the others bin the records. Neither needs anything of the
+// other.
+__global__ __launch_bounds__(256) void raster_bin_kernel(Workspace ws, uint2* entries,
+                                                         uint32_t capacity, int tile_blocks) {
+  __shared__ union {
+    TileStage place;
+    uint32_t filled[kStageTiles * kDepthSlabs];
+    TileTable table;
+  } lds;
+  // Entries beyond the buffer's capacity: the pass is left to a later launch with a larger
+  // buffer (the cursors stay untouched, so that launch places every entry).
+  if (ws.counters[1] > capacity) return;  // uniform over the grid
+  const int block = (int)blockIdx.x;
+  if (block < tile_blocks) {
+    place_tiles(ws, lds.place, block);
+    __syncthreads();  // its LDS becomes the counts of the large triangles
+    bin_large(ws, lds.filled, entries, block);
+  } else {
+    bin_records(ws, lds.table, entries, block - tile_blocks);
   }
 }
 
-// Pass 3, one thread per tile: its place in the order.
-__global__ __launch_bounds__(256) void raster_tile_place(Workspace ws) {
-  __shared__ uint32_t hist[kXcdShares * kWorkClasses];
-  __shared__ uint32_t base[kXcdShares * kWorkClasses];
-  for (int i = threadIdx.x; i < kXcdShares * kWorkClasses; i += blockDim.x) hist[i] = 0u;
-  __syncthreads();
-  const int64_t tile = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int slot = 0;
-  if (tile < ws.tiles) {
-    slot = xcd_share(tile, ws.tiles) * kWorkClasses + ws.tile_class[tile];
-    atomicAdd(hist + slot, 1u);
-  }
-  __syncthreads();
-  constexpr int kClassesPerThread = kXcdShares * kWorkClasses / 256;
-  uint32_t reserved[kClassesPerThread];
-#pragma unroll
-  for (int k = 0; k < kClassesPerThread; ++k) {
-    const int i = threadIdx.x + k * 256;
-    reserved[k] = hist[i] ? atomicAdd(ws.class_cursor + i, hist[i]) : 0u;
-  }
-#pragma unroll
-  for (int k = 0; k < kClassesPerThread; ++k) {
-    const int i = threadIdx.x + k * 256;
-    base[i] = reserved[k];
-    hist[i] = 0u;
-  }
-  __syncthreads();
-  if (tile < ws.tiles) ws.tile_order[base[slot] + atomicAdd(hist + slot, 1u)] = (uint32_t)tile;
+static void launch_bin(const Workspace& ws, uint2* entries, uint32_t capacity, hipStream_t s) {
+  const int record_blocks = (ws.record_blocks + kBinBlocks - 1) / kBinBlocks;
+  const int tile_blocks = blocks_for(ws.tiles, kStageTiles);
+  raster_bin_kernel<<<tile_blocks + record_blocks, 256, 0, s>>>(ws, entries, capacity,
+                                                                 tile_blocks);
 }
 
 // One workgroup per tile: the tile's keys stay in LDS while it walks the tile's binned
@@ -1248,7 +1356,7 @@ __device__ __forceinline__ void tile_pass(const DrRasterGeometry& g, const uint6
   for (uint32_t slot = blockIdx.x / kXcdShares; slot < busy; slot += stride) {
   const uint32_t tile = ws.tile_order[ws.share_info[kXcdShares + share] + slot];
   const uint32_t begin = ws.list_offsets[(size_t)tile * ws.slabs];
-  const uint32_t end = ws.list_offsets[(size_t)(tile + 1) * ws.slabs];
+  const uint32_t end = ws.list_cursor[(size_t)(tile + 1) * ws.slabs - 1];  // filled: its end
   if (begin == end) {  // uniform over the workgroup
     if (!kLoop) break;
     continue;
@@ -1851,15 +1959,10 @@ static int queue_visibility_start(const DrRasterGeometry* g, const uint64_t* pre
     }
     raster_setup_kernel<<<blocks_for(g->num_instances, 256), 256, 0, s>>>(*g, prev_keys, keys,
                                                                           ws, small_pixels(*g));
-    raster_scan_reduce<<<ws.scan_blocks, 256, 0, s>>>(ws.list_counts, ws.lists, ws.block_sums);
-    raster_scan_blocks<<<1, 256, 0, s>>>(ws.block_sums, ws.scan_blocks, ws.counters);
-    raster_scan_apply<<<ws.scan_blocks, 256, 0, s>>>(ws.list_counts, ws.lists, ws.block_sums,
-                                                     ws.list_offsets, ws.list_cursor,
-                                                     ws.chunk_offsets);
-    const int tile_blocks = blocks_for(ws.tiles, 256);
-    raster_tile_classes<<<tile_blocks, 256, 0, s>>>(ws);
-    raster_tile_cursors<<<1, 256, 0, s>>>(ws);
-    raster_tile_place<<<tile_blocks, 256, 0, s>>>(ws);
+    if (ws.slabs == 1)
+      raster_list_kernel<1><<<ws.list_blocks, kListThreads, 0, s>>>(ws);
+    else
+      raster_list_kernel<4><<<ws.list_blocks, kListThreads, 0, s>>>(ws);
   }
   const int status = launch_status();
   if (status != DR_OK) return status;
@@ -1913,7 +2016,7 @@ static int queue_visibility(const DrRasterGeometry* g, const uint64_t* prev_keys
   if ((int64_t)g->batch * g->height * g->width == 0 || g->num_instances == 0) return DR_OK;
   Workspace ws = layout(*g, (char*)workspace);
   if (capacity > 0) {
-    raster_bin_kernel<<<bin_grid(ws), 256, 0, s>>>(ws, entries, capacity);
+    launch_bin(ws, entries, capacity, s);
     launch_tile_pass(*g, prev_keys, keys, ws, entries, capacity, tile_groups, s);
   }
   raster_overflow_kernel<<<overflow_grid(ws), 256, 0, s>>>(*g, prev_keys, keys, ws, capacity);
@@ -2036,7 +2139,7 @@ extern "C" int dr_raster_visibility_bin(const DrRasterGeometry* g, void* workspa
   Workspace ws = layout(*g, (char*)workspace);
   if (!workspace || workspace_bytes < ws.bytes) return DR_ERR_CAPACITY;
   hipStream_t s = (hipStream_t)stream;
-  raster_bin_kernel<<<bin_grid(ws), 256, 0, s>>>(ws, (uint2*)entries, counts[1]);
+  launch_bin(ws, (uint2*)entries, counts[1], s);
   return launch_status();
 }
 

@@ -102,6 +102,33 @@ def test_mixed_triangle_sizes():
     assert_layers_match(pos, tri, (96, 80), count=2)
 
 
+@pytest.mark.parametrize("count,resolution,batch", [
+    (9, (97, 131), 1),     # one list workgroup, partial tiles
+    (300, (64, 64), 1),    # more large triangles than the list of them holds; depth slabs
+    (40, (1100, 252), 2),  # lists of several workgroups, tile rows split between them
+    (2000, (160, 176), 140),  # dense: only triangles over more than 64 tiles are large
+])
+def test_triangles_over_many_tiles(count, resolution, batch):
+    gen = torch.Generator().manual_seed(31)
+    pos, tri = random_mesh(count, gen, batch=min(batch, 2), xy_range=1.5)
+    if batch <= 2:
+        assert_layers_match(pos, tri, resolution, count=2)
+        return
+    pos = pos[torch.arange(batch) % 2].contiguous()
+    ours = gpu_layers(pos, tri, resolution, 2)
+    each = gpu_layers(pos[:2], tri, resolution, 2)  # few instances: large from 9 tiles
+    for (rast, db), (rast2, db2) in zip(ours, each):
+        assert torch.equal(rast, rast2[torch.arange(batch) % 2])
+        assert torch.equal(db, db2[torch.arange(batch) % 2])
+    assert_layers_match(pos[:1], tri, resolution)
+    # The same triangles as items of a range call (one list per tile).
+    ranges = torch.tensor([[0, 9], [9, 200], [500, 1500]], dtype=torch.int32)
+    flat = pos[0].cuda()
+    rast, _, _ = hip.rasterize_ranges(flat, tri.cuda(), resolution, True, ranges)
+    ref, _ = R.rasterize_ranges(pos[0], tri, resolution, ranges)
+    assert torch.equal(rast[..., 3].cpu(), ref[..., 3])
+
+
 def test_large_mesh_in_spatial_order_keeps_index_tie_break():
     # Meshes of 8192 triangles or more are processed in a spatially sorted order. Copies of
     # earlier triangles appended at the end tie in depth with their originals, which must win;

@@ -459,7 +459,7 @@ __device__ __forceinline__ int zw_tri(const DrAntialiasArgs& a, float2 zw, float
   return (id >= 1.0f && id <= (float)a.num_tri) ? (int)id - 1 : -1;
 }
 
-// The 16 x 16 tile of a pixel, numbered as tile_pixel() numbers workgroups before xcd_order.
+// The 16 x 16 tile of a pixel, numbered in image and row order.
 __device__ __forceinline__ int64_t tile_of(const DrAntialiasArgs& a, const TilePixel& tp) {
   const int tiles_x = (a.width + 15) / 16, tiles_y = (a.height + 15) / 16;
   return ((int64_t)tp.b * tiles_y + tp.y / 16) * tiles_x + tp.x / 16;

@@ -122,6 +122,7 @@ struct Workspace {
   int list_blocks;
   int record_blocks;          // setup workgroups; each owns 256 record slots
   int slabs;                  // tile lists per tile: kDepthSlabs, or 1 in range mode
+  uint32_t share_run;         // consecutive tiles of one XCD share of the tile pass
   uint32_t large_limit;       // a triangle over more tiles than this is a large one
   size_t bytes;
 };
@@ -155,6 +156,7 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
                                                                                   : kDepthSlabs;
   w.lists = w.tiles * w.slabs;
   w.large_limit = large_tiles_limit(g);
+  w.share_run = tile_run(g.batch, (uint32_t)std::min<int64_t>(w.tiles, 0xffffffffLL));
   const int64_t list_block = (int64_t)kListThreads * (w.slabs == 1 ? 1 : 4);
   w.list_blocks = (int)((w.lists + list_block - 1) / list_block);
   w.depth_ranges = (g.ranges == nullptr && g.pos_batch_stride != 0) ? std::max(g.batch, 1) : 1;
@@ -948,18 +950,14 @@ __global__ __launch_bounds__(256) void raster_setup_kernel(DrRasterGeometry g,
 // ---- kernels: tile lists ------------------------------------------------------------------
 //
 // The lists' places among the entries, and the tile pass's order: heavy tiles first within each
-// XCD's share. The tile pass takes the busy tiles in their XCD shares' order (so that XCD k,
-// which takes the k-th eighth of the workgroups under xcd_order, gets about share k), within a
-// share the tiles with the most binned triangles first, so that the longest workgroups do not
+// XCD's share. The tile pass takes the busy tiles in their XCD shares' order (its workgroups of
+// XCD k take share k), within a share the tiles with the most binned triangles first, so that the longest workgroups do not
 // start last: a counting sort by entry count in kWorkClasses classes of 32 entries. The order
 // within a class is free: tiles are independent.
 
-// The XCD share of tile i under xcd_order, and the first tile of share k.
-__device__ __forceinline__ int xcd_share(int64_t i, int64_t tiles) {
-  if (tiles < kXcdShares) return (int)i;
-  const int64_t per = tiles / kXcdShares, extra = tiles % kXcdShares;
-  const int64_t big = extra * (per + 1);
-  return i < big ? (int)(i / (per + 1)) : (int)(extra + (i - big) / per);
+// The XCD share of tile i: runs of tiles in turn (tile_run).
+__device__ __forceinline__ int xcd_share(const Workspace& ws, int64_t i) {
+  return (int)(((uint32_t)i / ws.share_run) % kXcdShares);
 }
 
 // Calls f(list - first_list, record, depth bound bits) for every tile list of
@@ -1056,7 +1054,7 @@ __global__ __launch_bounds__(kListThreads) void raster_list_kernel(Workspace ws)
     if (tile >= ws.tiles) return;
     const int c = n == 0 ? 0 : (int)min((n >> 5) + 1, (uint32_t)(kWorkClasses - 1));
     ws.tile_class[tile] = (uint8_t)c;
-    atomicAdd(s_hist + xcd_share(tile, ws.tiles) * kWorkClasses + c, 1u);
+    atomicAdd(s_hist + xcd_share(ws, tile) * kWorkClasses + c, 1u);
   };
   if constexpr (PER == 1) {
     classify(i0, total[0]);
@@ -1165,7 +1163,7 @@ __device__ __forceinline__ void place_tiles(const Workspace& ws, TileStage& p, i
   const int64_t tile = (int64_t)block * kStageTiles + threadIdx.x;
   int slot = 0;
   if (tile < ws.tiles) {
-    slot = xcd_share(tile, ws.tiles) * kWorkClasses + ws.tile_class[tile];
+    slot = xcd_share(ws, tile) * kWorkClasses + ws.tile_class[tile];
     atomicAdd(p.hist + slot, 1u);
   }
   __syncthreads();
@@ -1897,8 +1895,9 @@ extern "C" int dr_raster_workspace_size(const DrRasterGeometry* g, size_t* bytes
 // The tile pass's grid when the busy tiles are not known yet: 8 x the largest share of tiles
 // (its workgroups beyond a share's busy tiles return at once).
 static int64_t tile_grid_bound(const Workspace& ws) {
-  return ws.tiles < kXcdShares ? kXcdShares
-                               : kXcdShares * ((ws.tiles + kXcdShares - 1) / kXcdShares);
+  // Share 0 takes the most runs, each of at most share_run tiles (xcd_share).
+  const int64_t runs = (ws.tiles + ws.share_run - 1) / ws.share_run;
+  return kXcdShares * ((runs + kXcdShares - 1) / kXcdShares) * (int64_t)ws.share_run;
 }
 
 // The order passes, into ws.order (after raster_prepare has zeroed the bucket counts).
@@ -1978,8 +1977,8 @@ static int queue_visibility_start(const DrRasterGeometry* g, const uint64_t* pre
 constexpr int64_t kPlainTileGrid = 1 << 16;
 
 // Launches the tile pass so that it covers every busy tile whatever `requested` is. A grid of
-// at least one workgroup per tile (`requested` 0 or at least that, and then at most
-// kPlainTileGrid workgroups) runs the plain kernel, one tile per workgroup. Any smaller grid
+// at least one workgroup per tile of the largest share (`requested` 0 or at least 8 x that, and
+// then at most kPlainTileGrid tiles) runs the plain kernel, one tile per workgroup. Any smaller grid
 // runs the looping kernel: `requested` workgroups (0: one per tile), rounded up to a multiple
 // of 8 and kept below 2^24, each taking every (grid / 8)-th busy tile of its XCD share. So a
 // grid sized before the busy tiles were known, or sized wrongly by a caller, loses no tile.
@@ -1989,7 +1988,7 @@ static void launch_tile_pass(const DrRasterGeometry& g, const uint64_t* prev, ui
   const int64_t bound = tile_grid_bound(ws);
   const int64_t limit = ((int64_t)1 << 24) - kXcdShares;
   const bool full = requested == 0 || (int64_t)requested >= bound;
-  if (full && bound <= kPlainTileGrid) {
+  if (full && ws.tiles <= kPlainTileGrid) {
     raster_tile_kernel<false><<<(int)bound, 256, 0, s>>>(g, prev, keys, ws, entries, capacity);
     return;
   }

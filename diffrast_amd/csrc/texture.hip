@@ -349,23 +349,12 @@ struct MipLevels {
   int64_t off[DR_MAX_LEVELS];
 };
 
-// Level k + 1 from level k, one thread per destination texel and channel.
-__global__ __launch_bounds__(256) void mip_down(float* texels, int C, int64_t num_texels,
-                                                       int faces, MipLevels L, int k,
-                                                       int64_t count) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  const int h = L.h[k], w = L.w[k], h2 = L.h[k + 1], w2 = L.w[k + 1];
-  const int c = (int)(i % C);
-  int64_t rest = i / C;
-  const int col = (int)(rest % w2);
-  rest /= w2;
-  const int row = (int)(rest % h2);
-  rest /= h2;
-  const int face = (int)(rest % faces);
-  const int64_t image = rest / faces;
-  const float* src = texels + image * num_texels * C + (L.off[k] + (int64_t)face * h * w) * C;
-  float* dst = texels + image * num_texels * C + (L.off[k + 1] + (int64_t)face * h2 * w2) * C;
+// Value i of level k + 1 ((row, col, channel) order) from level k of one image and face.
+__device__ __forceinline__ void down_value(const float* src, float* dst, int C, int h, int w,
+                                           int w2, uint32_t i) {
+  const uint32_t texel = i / (uint32_t)C;
+  const int c = (int)(i - texel * (uint32_t)C);
+  const int row = (int)(texel / (uint32_t)w2), col = (int)(texel - (uint32_t)row * w2);
   int r0, nr, c0, nc;
   axis_taps(row, h, r0, nr);
   axis_taps(col, w, c0, nc);
@@ -377,28 +366,16 @@ __global__ __launch_bounds__(256) void mip_down(float* texels, int C, int64_t nu
       sum += (wr * wc) * src[((int64_t)(r0 + ri) * w + (c0 + ci)) * C + c];
     }
   }
-  dst[((int64_t)row * w2 + col) * C + c] = sum;
+  dst[(int64_t)i] = sum;
 }
 
-// Adjoint of mip_down: source texel (i, j) of level k gathers the gradient of the
-// destination texels of level k + 1 whose bins overlap it.
-__global__ __launch_bounds__(256) void mip_up(float* grad, int C, int64_t num_texels,
-                                                     int faces, MipLevels L, int k,
-                                                     int64_t count) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= count) return;
-  const int h = L.h[k], w = L.w[k], h2 = L.h[k + 1], w2 = L.w[k + 1];
-  const int c = (int)(idx % C);
-  int64_t rest = idx / C;
-  const int j = (int)(rest % w);
-  rest /= w;
-  const int i = (int)(rest % h);
-  rest /= h;
-  const int face = (int)(rest % faces);
-  const int64_t image = rest / faces;
-  float* src = grad + image * num_texels * C + (L.off[k] + (int64_t)face * h * w) * C;
-  const float* dst =
-      grad + image * num_texels * C + (L.off[k + 1] + (int64_t)face * h2 * w2) * C;
+// Adjoint of down_value: value idx of level k gathers the gradient of the texels of level k + 1
+// whose bins overlap it.
+__device__ __forceinline__ void up_value(float* src, const float* dst, int C, int h, int w,
+                                         int h2, int w2, uint32_t idx) {
+  const uint32_t texel = idx / (uint32_t)C;
+  const int c = (int)(idx - texel * (uint32_t)C);
+  const int i = (int)(texel / (uint32_t)w), j = (int)(texel - (uint32_t)i * w);
   // Destination rows (cols) that can overlap source row i (col j).
   const int r_mid = (h & 1) ? (int)((int64_t)i * h2 / h) : i / 2;
   const int c_mid = (w & 1) ? (int)((int64_t)j * w2 / w) : j / 2;
@@ -412,7 +389,76 @@ __global__ __launch_bounds__(256) void mip_up(float* grad, int C, int64_t num_te
       sum += (wr * wc) * dst[((int64_t)r * w2 + cc) * C + c];
     }
   }
-  src[((int64_t)i * w + j) * C + c] += sum;
+  src[(int64_t)idx] += sum;
+}
+
+// Level lvl of (image, face) number `face_of`, image by image.
+__device__ __forceinline__ float* level_of(float* texels, int64_t num_texels, int C,
+                                           const MipLevels& L, int lvl, int64_t image, int face) {
+  return texels + image * num_texels * C +
+         (L.off[lvl] + (int64_t)face * L.h[lvl] * L.w[lvl]) * C;
+}
+
+// Level k + 1 from level k, one thread per destination texel and channel, `blocks` workgroups
+// per (image, face).
+__global__ __launch_bounds__(256) void mip_down(float* texels, int C, int64_t num_texels,
+                                                int faces, MipLevels L, int k, uint32_t blocks) {
+  const uint32_t which = blockIdx.x / blocks;
+  const uint32_t i = (blockIdx.x - which * blocks) * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)L.h[k + 1] * L.w[k + 1] * C) return;
+  const int64_t image = which / (uint32_t)faces;
+  const int face = (int)(which % (uint32_t)faces);
+  down_value(level_of(texels, num_texels, C, L, k, image, face),
+             level_of(texels, num_texels, C, L, k + 1, image, face), C, L.h[k], L.w[k],
+             L.w[k + 1], i);
+}
+
+// Adjoint of mip_down: one thread per source texel and channel.
+__global__ __launch_bounds__(256) void mip_up(float* grad, int C, int64_t num_texels, int faces,
+                                              MipLevels L, int k, uint32_t blocks) {
+  const uint32_t which = blockIdx.x / blocks;
+  const uint32_t i = (blockIdx.x - which * blocks) * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)L.h[k] * L.w[k] * C) return;
+  const int64_t image = which / (uint32_t)faces;
+  const int face = (int)(which % (uint32_t)faces);
+  up_value(level_of(grad, num_texels, C, L, k, image, face),
+           level_of(grad, num_texels, C, L, k + 1, image, face), C, L.h[k], L.w[k], L.h[k + 1],
+           L.w[k + 1], i);
+}
+
+// Levels k + 1 .. last from level k, one workgroup per (image, face): for levels so small that
+// a launch each would be nearly all launch (kMipTailValues values). Odd sizes included.
+constexpr int kMipTailThreads = 1024;
+
+__global__ __launch_bounds__(kMipTailThreads) void mip_down_tail(float* texels, int C,
+                                                                 int64_t num_texels, int faces,
+                                                                 MipLevels L, int k, int last) {
+  const int64_t image = blockIdx.x / (uint32_t)faces;
+  const int face = (int)(blockIdx.x % (uint32_t)faces);
+  for (int lvl = k; lvl < last; ++lvl) {
+    const float* src = level_of(texels, num_texels, C, L, lvl, image, face);
+    float* dst = level_of(texels, num_texels, C, L, lvl + 1, image, face);
+    const uint32_t count = (uint32_t)(L.h[lvl + 1] * L.w[lvl + 1] * C);
+    for (uint32_t i = threadIdx.x; i < count; i += kMipTailThreads)
+      down_value(src, dst, C, L.h[lvl], L.w[lvl], L.w[lvl + 1], i);
+    __syncthreads();  // the next level reads what the workgroup wrote
+  }
+}
+
+// Adjoint of mip_down_tail.
+__global__ __launch_bounds__(kMipTailThreads) void mip_up_tail(float* grad, int C,
+                                                               int64_t num_texels, int faces,
+                                                               MipLevels L, int k, int last) {
+  const int64_t image = blockIdx.x / (uint32_t)faces;
+  const int face = (int)(blockIdx.x % (uint32_t)faces);
+  for (int lvl = last - 1; lvl >= k; --lvl) {
+    float* src = level_of(grad, num_texels, C, L, lvl, image, face);
+    const float* dst = level_of(grad, num_texels, C, L, lvl + 1, image, face);
+    const uint32_t count = (uint32_t)(L.h[lvl] * L.w[lvl] * C);
+    for (uint32_t i = threadIdx.x; i < count; i += kMipTailThreads)
+      up_value(src, dst, C, L.h[lvl], L.w[lvl], L.h[lvl + 1], L.w[lvl + 1], i);
+    __syncthreads();  // the next level reads what the workgroup wrote
+  }
 }
 
 // ---- mip chain in tile stages ------------------------------------------------------------
@@ -430,34 +476,42 @@ __global__ __launch_bounds__(256) void mip_up(float* grad, int C, int64_t num_te
 // folded back, 63 -> 53 us; tiles of 16 x 16 need a third stage, 66 us.)
 constexpr int kMipStageLevels = 5;
 
-// Up to four channels of texel p (n valid; vec: four channels on a 16-byte aligned buffer).
-__device__ __forceinline__ float4 load_texel(const float* p, int n, bool vec) {
-  if (vec) return *reinterpret_cast<const float4*>(p);
-  return make_float4(p[0], n > 1 ? p[1] : 0.f, n > 2 ? p[2] : 0.f, n > 3 ? p[3] : 0.f);
+// The stages work on elements of a texel: float4 when the channels come in fours on a 16-byte
+// aligned buffer, else single channels. Consecutive lanes take a texel's elements in turn, so
+// that a wave's loads cover whole lines whatever the channel count (one lane per texel and
+// group of four, a pass per group, at 1024^2 x 16: 199 us to build the chain and 178 to fold
+// it; now 37 and 44).
+__device__ __forceinline__ float quad_mean(float a, float b, float c, float d) {
+  return ((0.25f * a + 0.25f * b) + 0.25f * c) + 0.25f * d;
 }
-
-__device__ __forceinline__ void store_texel(float* p, float4 v, int n, bool vec) {
-  if (vec) {
-    *reinterpret_cast<float4*>(p) = v;
-    return;
-  }
-  p[0] = v.x;
-  if (n > 1) p[1] = v.y;
-  if (n > 2) p[2] = v.z;
-  if (n > 3) p[3] = v.w;
-}
-
 __device__ __forceinline__ float4 quad_mean(float4 a, float4 b, float4 c, float4 d) {
-  auto mean = [](float a, float b, float c, float d) {
-    return ((0.25f * a + 0.25f * b) + 0.25f * c) + 0.25f * d;
-  };
-  return make_float4(mean(a.x, b.x, c.x, d.x), mean(a.y, b.y, c.y, d.y),
-                     mean(a.z, b.z, c.z, d.z), mean(a.w, b.w, c.w, d.w));
+  return make_float4(quad_mean(a.x, b.x, c.x, d.x), quad_mean(a.y, b.y, c.y, d.y),
+                     quad_mean(a.z, b.z, c.z, d.z), quad_mean(a.w, b.w, c.w, d.w));
+}
+__device__ __forceinline__ float add_quarter(float own, float parent) {
+  return own + 0.25f * parent;
+}
+__device__ __forceinline__ float4 add_quarter(float4 own, float4 parent) {
+  return make_float4(add_quarter(own.x, parent.x), add_quarter(own.y, parent.y),
+                     add_quarter(own.z, parent.z), add_quarter(own.w, parent.w));
 }
 
-__device__ __forceinline__ float4 add_quarter(float4 own, float4 parent) {
-  return make_float4(own.x + 0.25f * parent.x, own.y + 0.25f * parent.y,
-                     own.z + 0.25f * parent.z, own.w + 0.25f * parent.w);
+// Elements of a texel that a stage takes at a time (LDS: 20 KB), and the LDS of the levels of a
+// tile 2^j texels across: even j in one buffer (at most 16 x 16), odd j in the other (8 x 8).
+template <class V>
+constexpr int kStageElements = 64 / (int)sizeof(V);
+template <class V>
+struct MipStage {
+  V even[256 * kStageElements<V>], odd[64 * kStageElements<V>];
+  __device__ __forceinline__ V* side(int j) { return (j & 1) ? odd : even; }
+};
+
+// (texel, element) of a stage's element i, for NE elements per texel (0: ne, at run time).
+template <int NE>
+__device__ __forceinline__ void stage_element(int i, int ne, int& texel, int& e) {
+  const uint32_t n = NE > 0 ? (uint32_t)NE : (uint32_t)ne;
+  texel = (int)((uint32_t)i / n);
+  e = i - texel * (int)n;
 }
 
 // The tile of this workgroup: (image, face) and tile coordinates in units of 2^G bottom texels.
@@ -479,120 +533,178 @@ __device__ __forceinline__ MipTile mip_tile(const MipLevels& L, int k, int G, in
   return T;
 }
 
-__device__ __forceinline__ float* mip_level(float* texels, int64_t num_texels, int C,
-                                            const MipLevels& L, const MipTile& T, int lvl) {
-  return texels + T.image * num_texels * C + (L.off[lvl] + (int64_t)T.face * L.h[lvl] * L.w[lvl]) * C;
-}
-
 // Levels k + 1 .. k + G from level k, one tile per workgroup. With `base` (k == 0 only), level
 // 0 is read from there -- [images, faces * h * w, C], the layout of level 0 on its own -- and
-// copied into the packed buffer on the way (each of its texels is read once).
-__global__ __launch_bounds__(256) void mip_down_stage(float* texels, const float* base, int C,
+// copied into the packed buffer on the way (each of its texels is read once). E: elements per
+// texel, C in elements of type V.
+template <class V, int NE>
+__global__ __launch_bounds__(256) void mip_down_stage(V* texels, const V* base, int E,
                                                       int64_t num_texels, int faces,
                                                       MipLevels L, int k, int G) {
-  __shared__ float4 s_buf[2][1 << (2 * kMipStageLevels - 2)];
+  __shared__ MipStage<V> stage;
   const MipTile T = mip_tile(L, k, G, faces);
-  const bool vec = C == 4 && (reinterpret_cast<uintptr_t>(texels) & 15u) == 0 &&
-                   (reinterpret_cast<uintptr_t>(base) & 15u) == 0;
-  for (int c0 = 0; c0 < C; c0 += 4) {
-    const int n = min(4, C - c0);
-    int side = 1 << (G - 1);  // the tile's side at level k + 1
+  auto level_at = [&](int lvl) {
+    return texels + (T.image * num_texels + L.off[lvl] + (int64_t)T.face * L.h[lvl] * L.w[lvl]) * E;
+  };
+  for (int e0 = 0; e0 < E; e0 += kStageElements<V>) {
+    const int ne = min(kStageElements<V>, E - e0);
     {
-      float* level = mip_level(texels, num_texels, C, L, T, k) + c0;
-      const float* src =
-          base ? base + (T.image * faces + T.face) * (int64_t)L.h[0] * L.w[0] * C + c0 : level;
-      float* dst = mip_level(texels, num_texels, C, L, T, k + 1) + c0;
-      const int64_t w = L.w[k], w1 = L.w[k + 1];
-      for (int i = threadIdx.x; i < side * side; i += blockDim.x) {
-        const int r = T.ty * side + i / side, c = T.tx * side + i % side;
-        const int64_t at = ((int64_t)(2 * r) * w + 2 * c) * C;
-        const float* p = src + at;
-        const float4 a = load_texel(p, n, vec), b = load_texel(p + C, n, vec);
-        const float4 cc = load_texel(p + w * C, n, vec), d = load_texel(p + w * C + C, n, vec);
+      const int j = G - 1, side = 1 << j;  // the tile's side at level k + 1
+      V* level = level_at(k) + e0;
+      const V* src =
+          base ? base + (T.image * faces + T.face) * (int64_t)L.h[0] * L.w[0] * E + e0 : level;
+      V* dst = level_at(k + 1) + e0;
+      const int64_t w = (int64_t)L.w[k] * E, w1 = (int64_t)L.w[k + 1] * E;
+      V* out = stage.side(j);
+#pragma unroll 2
+      for (int i = threadIdx.x; i < side * side * ne; i += blockDim.x) {
+        int texel, e;
+        stage_element<NE>(i, ne, texel, e);
+        const int r = T.ty * side + (texel >> j), c = T.tx * side + (texel & (side - 1));
+        const int64_t at = 2 * r * w + (int64_t)(2 * c) * E + e;
+        const V* p = src + at;
+        const V v00 = p[0], v01 = p[E], v10 = p[w], v11 = p[w + E];
         if (base) {
-          float* q = level + at;
-          store_texel(q, a, n, vec);
-          store_texel(q + C, b, n, vec);
-          store_texel(q + w * C, cc, n, vec);
-          store_texel(q + w * C + C, d, n, vec);
+          V* q = level + at;
+          q[0] = v00;
+          q[E] = v01;
+          q[w] = v10;
+          q[w + E] = v11;
         }
-        const float4 o = quad_mean(a, b, cc, d);
-        store_texel(dst + ((int64_t)r * w1 + c) * C, o, n, vec);
-        s_buf[0][i] = o;
+        const V o = quad_mean(v00, v01, v10, v11);
+        dst[r * w1 + (int64_t)c * E + e] = o;
+        out[i] = o;
       }
     }
-    int cur = 0;
     for (int lvl = k + 2; lvl <= k + G; ++lvl) {
       __syncthreads();
-      const int below = side;
-      side >>= 1;
-      float* dst = mip_level(texels, num_texels, C, L, T, lvl) + c0;
-      const int64_t wl = L.w[lvl];
-      const float4* s = s_buf[cur];
-      for (int i = threadIdx.x; i < side * side; i += blockDim.x) {
-        const int r = i / side, c = i % side;
-        const float4* q = s + 2 * r * below + 2 * c;
-        const float4 o = quad_mean(q[0], q[1], q[below], q[below + 1]);
-        store_texel(dst + ((int64_t)(T.ty * side + r) * wl + T.tx * side + c) * C, o, n, vec);
-        s_buf[cur ^ 1][i] = o;
+      const int j = k + G - lvl, side = 1 << j;
+      const V* s = stage.side(j + 1);
+      V* out = stage.side(j);
+      V* dst = level_at(lvl) + e0;
+      const int64_t wl = (int64_t)L.w[lvl] * E;
+      for (int i = threadIdx.x; i < side * side * ne; i += blockDim.x) {
+        int texel, e;
+        stage_element<NE>(i, ne, texel, e);
+        const int r = texel >> j, c = texel & (side - 1);
+        const V* q = s + ((2 * r * 2 * side) + 2 * c) * ne + e;
+        const V o = quad_mean(q[0], q[ne], q[2 * side * ne], q[(2 * side + 1) * ne]);
+        dst[(T.ty * side + r) * wl + (int64_t)(T.tx * side + c) * E + e] = o;
+        out[i] = o;
       }
-      cur ^= 1;
     }
-    __syncthreads();  // the next channel group reuses the LDS
+    __syncthreads();  // the next elements reuse the LDS
   }
 }
 
 // Adjoint of mip_down_stage: the totals of level k + G (final: the stages above ran first) fold
 // down through levels k + G - 1 .. k of the tile, each texel adding a quarter of its parent's
 // total to its own gradient, which becomes its total.
-__global__ __launch_bounds__(256) void mip_up_stage(float* grad, int C, int64_t num_texels,
-                                                    int faces, MipLevels L, int k, int G) {
-  __shared__ float4 s_buf[2][1 << (2 * kMipStageLevels - 2)];
+template <class V, int NE>
+__global__ __launch_bounds__(256) void mip_up_stage(V* grad, int E, int64_t num_texels, int faces,
+                                                    MipLevels L, int k, int G) {
+  __shared__ MipStage<V> stage;
   const MipTile T = mip_tile(L, k, G, faces);
-  const bool vec = C == 4 && (reinterpret_cast<uintptr_t>(grad) & 15u) == 0;
-  for (int c0 = 0; c0 < C; c0 += 4) {
-    const int n = min(4, C - c0);
-    int cur = 0;
-    if (threadIdx.x == 0) {
-      const float* top = mip_level(grad, num_texels, C, L, T, k + G) + c0;
-      s_buf[0][0] = load_texel(top + ((int64_t)T.ty * L.w[k + G] + T.tx) * C, n, vec);
-    }
-    int side = 1;  // the tile's side at the level in s_buf[cur]
+  auto level_at = [&](int lvl) {
+    return grad + (T.image * num_texels + L.off[lvl] + (int64_t)T.face * L.h[lvl] * L.w[lvl]) * E;
+  };
+  for (int e0 = 0; e0 < E; e0 += kStageElements<V>) {
+    const int ne = min(kStageElements<V>, E - e0);
+    if ((int)threadIdx.x < ne)
+      stage.side(0)[threadIdx.x] =
+          level_at(k + G)[((int64_t)T.ty * L.w[k + G] + T.tx) * E + e0 + threadIdx.x];
     for (int lvl = k + G - 1; lvl >= k; --lvl) {
       __syncthreads();
-      const int above = side;
-      side <<= 1;
-      float* g = mip_level(grad, num_texels, C, L, T, lvl) + c0;
-      const int64_t wl = L.w[lvl];
-      const float4* s = s_buf[cur];
-      for (int i = threadIdx.x; i < side * side; i += blockDim.x) {
-        const int r = i / side, c = i % side;
-        float* p = g + ((int64_t)(T.ty * side + r) * wl + T.tx * side + c) * C;
-        const float4 o = add_quarter(load_texel(p, n, vec), s[(r >> 1) * above + (c >> 1)]);
-        store_texel(p, o, n, vec);
-        if (lvl > k) s_buf[cur ^ 1][i] = o;
+      const int j = k + G - lvl, side = 1 << j;
+      const V* s = stage.side(j - 1);
+      V* out = stage.side(j);
+      V* g = level_at(lvl) + e0;
+      const int64_t wl = (int64_t)L.w[lvl] * E;
+      // Four elements per thread and step, all loaded before the first is stored (the stores
+      // go to the buffer the loads read: nothing else would keep the loads together).
+      constexpr int kStep = 4;
+      const int count = side * side * ne;
+      for (int i0 = threadIdx.x; i0 < count; i0 += kStep * 256) {
+        V own[kStep];
+        V* at[kStep];
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) {
+          const int i = min(i0 + 256 * u, count - 1);
+          int texel, e;
+          stage_element<NE>(i, ne, texel, e);
+          const int r = texel >> j, c = texel & (side - 1);
+          at[u] = g + (T.ty * side + r) * wl + (int64_t)(T.tx * side + c) * E + e;
+          own[u] = *at[u];
+        }
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) {
+          const int i = i0 + 256 * u;
+          if (i >= count) break;
+          int texel, e;
+          stage_element<NE>(i, ne, texel, e);
+          const int r = texel >> j, c = texel & (side - 1);
+          const V o = add_quarter(own[u], s[((r >> 1) * (side >> 1) + (c >> 1)) * ne + e]);
+          *at[u] = o;
+          if (lvl > k) out[i] = o;
+        }
       }
-      cur ^= 1;
     }
-    __syncthreads();  // the next channel group reuses the LDS
+    __syncthreads();  // the next elements reuse the LDS
   }
 }
 
-// Tile stages and single levels of a chain: stage (k, G) builds levels k + 1 .. k + G, in one
-// tile-stage launch when G >= 2, else (G == 1) with mip_down.
+// Calls f(element type tag, elements per texel as a constant (0: at run time)) for C channels at
+// the given buffers.
+template <typename F>
+void stage_elements(int C, const void* texels, const void* base, F f) {
+  using std::integral_constant;
+  const bool wide = C % 4 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(texels) | reinterpret_cast<uintptr_t>(base)) &
+                     15u) == 0;
+  if (wide) {
+    switch (C) {
+      case 4: return f(float4(), integral_constant<int, 1>());
+      case 8: return f(float4(), integral_constant<int, 2>());
+      default:  // a whole number of full passes, or the count at run time
+        return C % 16 == 0 ? f(float4(), integral_constant<int, 4>())
+                           : f(float4(), integral_constant<int, 0>());
+    }
+  }
+  switch (C) {
+    case 1: return f(float(), integral_constant<int, 1>());
+    case 2: return f(float(), integral_constant<int, 2>());
+    case 3: return f(float(), integral_constant<int, 3>());
+    default: return f(float(), integral_constant<int, 0>());
+  }
+}
+
+// Up to this many values of a level (per image and face), the rest of the chain is one
+// workgroup's: it takes 4 values per thread at a time, in about a launch's time each (limits of
+// 2048 to 16384 within 3 % of a step of 1500 x 1500 x 16: 722, 720 and 740 us).
+constexpr int64_t kMipTailValues = 4096;
+
+// Parts of a chain: part (k, G) builds levels k + 1 .. k + G, in one tile-stage launch when
+// G >= 2, else (G == 1) with mip_down; the part at index `tail`, if any, is the last, with
+// mip_down_tail.
 struct MipPlan {
   int count;
+  int tail;
   int k[DR_MAX_LEVELS], G[DR_MAX_LEVELS];
 };
 
-MipPlan mip_plan(const MipLevels& L, int num_levels) {
+MipPlan mip_plan(const MipLevels& L, int num_levels, int channels) {
   MipPlan P{};
+  P.tail = -1;
   for (int k = 0; k + 1 < num_levels;) {
     int G = 0;
     while (G < kMipStageLevels && k + G + 1 < num_levels && L.h[k] % (2 << G) == 0 &&
            L.w[k] % (2 << G) == 0)
       ++G;
     if (G < 2) G = 1;
+    if (k + G + 1 < num_levels && (int64_t)L.h[k] * L.w[k] * channels <= kMipTailValues) {
+      P.tail = P.count;  // more than one launch otherwise
+      G = num_levels - 1 - k;
+    }
     P.k[P.count] = k;
     P.G[P.count] = G;
     ++P.count;
@@ -732,12 +844,12 @@ extern "C" int dr_mip_build(float* texels, const float* base, int32_t tex_batch,
       !valid_levels(num_levels, level_height, level_width, level_offset))
     return DR_ERR_ARGUMENT;
   const MipLevels L = copy_levels(num_levels, level_height, level_width, level_offset);
-  const MipPlan P = mip_plan(L, num_levels);
+  const MipPlan P = mip_plan(L, num_levels, channels);
   const int64_t images = (int64_t)tex_batch * faces;
   const int64_t base_texels = (int64_t)faces * L.h[0] * L.w[0];
   if (base != nullptr && base_texels > num_texels) return DR_ERR_ARGUMENT;
   // Level 0 from `base`: the first tile stage copies it as it reads it; otherwise a copy first.
-  const bool staged_copy = base != nullptr && P.count > 0 && P.G[0] >= 2;
+  const bool staged_copy = base != nullptr && P.count > 0 && P.G[0] >= 2 && P.tail != 0;
   if (base != nullptr && !staged_copy) {
     const int64_t count = (int64_t)tex_batch * base_texels * channels;
     mip_copy_base<<<blocks_for(count, 256), 256, 0, (hipStream_t)stream>>>(
@@ -745,14 +857,25 @@ extern "C" int dr_mip_build(float* texels, const float* base, int32_t tex_batch,
   }
   for (int s = 0; s < P.count; ++s) {
     const int k = P.k[s], G = P.G[s];
-    if (G >= 2) {
-      mip_down_stage<<<(unsigned)stage_tiles(L, k, G, images), 256, 0, (hipStream_t)stream>>>(
-          texels, s == 0 && staged_copy ? base : nullptr, channels, num_texels, faces, L, k, G);
+    if (s == P.tail) {
+      mip_down_tail<<<(unsigned)images, kMipTailThreads, 0, (hipStream_t)stream>>>(
+          texels, channels, num_texels, faces, L, k, k + G);
       continue;
     }
-    const int64_t count = images * L.h[k + 1] * L.w[k + 1] * channels;
-    mip_down<<<blocks_for(count, 256), 256, 0, (hipStream_t)stream>>>(
-        texels, channels, num_texels, faces, L, k, count);
+    if (G >= 2) {
+      const float* from = s == 0 && staged_copy ? base : nullptr;
+      stage_elements(channels, texels, from, [&](auto v, auto ne) {
+        using V = decltype(v);
+        mip_down_stage<V, decltype(ne)::value>
+            <<<(unsigned)stage_tiles(L, k, G, images), 256, 0, (hipStream_t)stream>>>(
+                (V*)texels, (const V*)from, channels / (int)(sizeof(V) / 4), num_texels, faces, L,
+                k, G);
+      });
+      continue;
+    }
+    const int64_t blocks = blocks_for((int64_t)L.h[k + 1] * L.w[k + 1] * channels, 256);
+    mip_down<<<(unsigned)(images * blocks), 256, 0, (hipStream_t)stream>>>(
+        texels, channels, num_texels, faces, L, k, (uint32_t)blocks);
   }
   return launch_status();
 }
@@ -765,18 +888,27 @@ extern "C" int dr_mip_build_backward(float* grad_texels, int32_t tex_batch, int3
       !valid_levels(num_levels, level_height, level_width, level_offset))
     return DR_ERR_ARGUMENT;
   const MipLevels L = copy_levels(num_levels, level_height, level_width, level_offset);
-  const MipPlan P = mip_plan(L, num_levels);
+  const MipPlan P = mip_plan(L, num_levels, channels);
   const int64_t images = (int64_t)tex_batch * faces;
   for (int s = P.count - 1; s >= 0; --s) {
     const int k = P.k[s], G = P.G[s];
-    if (G >= 2) {
-      mip_up_stage<<<(unsigned)stage_tiles(L, k, G, images), 256, 0, (hipStream_t)stream>>>(
-          grad_texels, channels, num_texels, faces, L, k, G);
+    if (s == P.tail) {
+      mip_up_tail<<<(unsigned)images, kMipTailThreads, 0, (hipStream_t)stream>>>(
+          grad_texels, channels, num_texels, faces, L, k, k + G);
       continue;
     }
-    const int64_t count = images * L.h[k] * L.w[k] * channels;
-    mip_up<<<blocks_for(count, 256), 256, 0, (hipStream_t)stream>>>(
-        grad_texels, channels, num_texels, faces, L, k, count);
+    if (G >= 2) {
+      stage_elements(channels, grad_texels, nullptr, [&](auto v, auto ne) {
+        using V = decltype(v);
+        mip_up_stage<V, decltype(ne)::value>
+            <<<(unsigned)stage_tiles(L, k, G, images), 256, 0, (hipStream_t)stream>>>(
+                (V*)grad_texels, channels / (int)(sizeof(V) / 4), num_texels, faces, L, k, G);
+      });
+      continue;
+    }
+    const int64_t blocks = blocks_for((int64_t)L.h[k] * L.w[k] * channels, 256);
+    mip_up<<<(unsigned)(images * blocks), 256, 0, (hipStream_t)stream>>>(
+        grad_texels, channels, num_texels, faces, L, k, (uint32_t)blocks);
   }
   return launch_status();
 }

@@ -4,6 +4,7 @@ Forward values within 1e-5 relative (normalised by max(|value|, 1)), gradients w
 (normalised by the largest reference gradient), both stated per test.
 """
 
+import math
 from pathlib import Path
 
 import numpy as np
@@ -331,6 +332,32 @@ def test_mip_chain_tile_stages(shape):
         t = tex.clone().to(device).requires_grad_(True)
         sum((l * w.to(device)).sum() for l, w in zip(fn(t, None), weights)).backward()
         grads.append(t.grad.cpu())
+    torch.testing.assert_close(grads[0], grads[1], atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("shape,offset", [
+    ((1, 64, 64, 16), 0), ((2, 64, 32, 20), 0),  # whole passes of channels, and a partial one
+    ((1, 64, 64, 8), 1),                         # the same on a buffer that is not aligned
+    ((1, 96, 96, 5), 0), ((2, 32, 32, 17), 0),   # channels that do not come in fours
+    ((3, 45, 30, 2), 0), ((1, 6, 24, 24, 3), 0),  # chains ending in one workgroup's levels
+    ((1, 130, 70, 7), 0),                        # levels of their own before those
+])
+def test_mip_chain_channels_and_tails(shape, offset):
+    gen = torch.Generator().manual_seed(6)
+    flat = torch.randn(math.prod(shape) + offset, generator=gen)
+    tex = flat[offset:].view(shape)
+    ref = R.texture_construct_mip(tex, None)
+    weights = [torch.randn(l.shape, generator=gen) for l in ref]
+    grads = []
+    for fn, device in ((hip.texture_construct_mip, "cuda"), (R.texture_construct_mip, "cpu")):
+        whole = flat.to(device).requires_grad_(True)
+        levels = fn(whole[offset:].view(shape), None)
+        for a, b in zip(levels, ref):
+            assert a.shape == b.shape
+            assert rel_error(a.detach().cpu(), b) < VALUE_TOL
+        sum((l * w.to(device)).sum() for l, w in zip(levels, weights)).backward()
+        grads.append(whole.grad.cpu())
+    # A base texel sums at most one product per level and axis weight: a few roundings.
     torch.testing.assert_close(grads[0], grads[1], atol=1e-5, rtol=1e-5)
 
 

@@ -68,6 +68,34 @@ def test_interpolate_forward_is_bit_exact(channels, layout):
         assert torch.equal(out[1].cpu(), ref[1])
 
 
+@pytest.mark.parametrize("channels,offset", [(6, 0), (7, 0), (12, 0), (12, 1), (10, 1), (259, 0),
+                                             (1028, 0)])
+@pytest.mark.parametrize("triangles", [80, 400_000])  # rows, and tiles (index rows beyond 4 MiB)
+def test_interpolate_many_channels(channels, offset, triangles):
+    # One, two or four channels per lane by count and alignment, more channels than a workgroup
+    # has lanes, tiles that show nothing (the left half of the image) and partial tiles.
+    gen = torch.Generator().manual_seed(8)
+    pos, tri = random_mesh(80, gen, batch=2)
+    pos[..., 0] = pos[..., 0].abs()
+    rast, rast_db = R.rasterize(pos, tri, (19, 70), True)
+    tri = torch.cat([tri, tri[:1].expand(triangles - 80, 3)])
+    v = pos.shape[1]
+    flat = torch.randn(v * channels + offset, generator=gen)
+    for diff in ([], [channels - 1, 0, 3]):
+        def run(fn, device):
+            whole = flat.clone().to(device).requires_grad_(True)
+            r, d = (t.detach().clone().to(device).requires_grad_(True)
+                    for t in (rast, rast_db))
+            out = fn(whole[offset:].view(v, channels), r, tri.to(device), d if diff else None,
+                     diff)
+            weight = torch.randn(out[0].shape, generator=torch.Generator().manual_seed(9))
+            (out[0] * weight.to(device)).sum().backward()
+            return [t.detach().cpu() for t in (*out, whole.grad, r.grad)]
+        ours, ref = run(hip.interpolate, "cuda"), run(R.interpolate, "cpu")
+        assert torch.equal(ours[0], ref[0]) and torch.equal(ours[1], ref[1])
+        assert_grads_close(ours[2:], ref[2:])
+
+
 @pytest.mark.parametrize("layout", ["shared", "per_view"])
 @pytest.mark.parametrize("diff", [[], [0, 2, 3], [1, 1]])
 def test_interpolate_gradients(layout, diff):

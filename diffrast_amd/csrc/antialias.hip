@@ -640,14 +640,13 @@ __device__ __forceinline__ PixelPairs pixel_pairs(const DrAntialiasArgs& a, cons
   return P;
 }
 
-// Channels [c0, c0 + n) of a pixel whose first channel is at p (n <= N; 0 past n): the widest
-// loads the alignment allows, all issued together.
+// Channels [c0, c0 + n) of a pixel whose first channel is at p (n <= N, uniform; 0 past n), all
+// loads issued together.
 template <int N>
 __device__ __forceinline__ void load_group(const float* p, int n, float (&v)[N]) {
-  if constexpr (N == 4) {
-    if (n == 4 && load_wide<4>(p, v)) return;
-  } else if constexpr (N == 2) {
-    if (n == 2 && load_wide<2>(p, v)) return;
+  if (n == N) {
+    load_floats(p, v);
+    return;
   }
 #pragma unroll
   for (int c = 0; c < N; ++c) v[c] = c < n ? p[c] : 0.0f;
@@ -655,8 +654,9 @@ __device__ __forceinline__ void load_group(const float* p, int n, float (&v)[N])
 
 template <int N>
 __device__ __forceinline__ void store_group(float* p, int n, const float (&v)[N]) {
-  if constexpr (N == 4 || N == 2) {
-    if (n == N && store_wide<N>(p, v)) return;
+  if (n == N) {
+    store_floats(p, v);
+    return;
   }
 #pragma unroll
   for (int c = 0; c < N; ++c)
@@ -666,14 +666,15 @@ __device__ __forceinline__ void store_group(float* p, int n, const float (&v)[N]
 // out = colour + |t - 0.5| of the neighbour's colour on the side of each crossing
 // (reference.py:253-264). A pixel takes (0.5 - t) of its pair partner when it is the first
 // pixel and t < 0.5, and (t - 0.5) when it is the second and t >= 0.5.
-// NC channels per group: the channel count for 1 to 4 channels (whole-pixel loads and stores),
-// 4 with a loop over groups for more.
-template <int NC, bool SPARSE>
+// CHANNELS: the channel count for 1 to 4 channels (whole-pixel loads and stores), 0 for more, in
+// groups of 4.
+template <int CHANNELS, bool SPARSE>
 __global__ __launch_bounds__(256) void aa_blend_kernel(DrAntialiasArgs a, const float2* pair_t,
                                                        const uchar2* pair_bits,
                                                        const uint8_t* tile_active, float* out) {
+  constexpr int NC = CHANNELS == 0 ? 4 : CHANNELS;
   const TilePixel tp = tile_pixel(a.batch, a.height, a.width);
-  const int C = a.channels;
+  const int C = CHANNELS > 0 ? CHANNELS : a.channels;
   const TileFlags flags = SPARSE ? tile_flags(a, tp, tile_active) : TileFlags{true, true, true};
   if (SPARSE && !flags.any()) {  // uniform: no pair moves colour here
     copy_tile(a, tp, a.color, out);
@@ -723,7 +724,7 @@ __global__ __launch_bounds__(256) void aa_blend_kernel(DrAntialiasArgs a, const 
 
 // Colour gradient (a gather over the same pairs) and position gradient of each active pair,
 // written by its first pixel through the workgroup's scatter table (rows of pos: x, y, z, w).
-template <int NC, bool SPARSE>
+template <int CHANNELS, bool SPARSE>
 __global__ __launch_bounds__(256) void aa_bwd_kernel(DrAntialiasArgs a, const float2* pair_t,
                                                      const uchar2* pair_bits,
                                                      const uint8_t* tile_active,
@@ -732,8 +733,9 @@ __global__ __launch_bounds__(256) void aa_bwd_kernel(DrAntialiasArgs a, const fl
   using Table = RowTable<512, 4>;
   __shared__ Table table;
   if (!SPARSE) table.init();
+  constexpr int NC = CHANNELS == 0 ? 4 : CHANNELS;
   const TilePixel tp = tile_pixel(a.batch, a.height, a.width);
-  const int C = a.channels;
+  const int C = CHANNELS > 0 ? CHANNELS : a.channels;
   const TileFlags flags = SPARSE ? tile_flags(a, tp, tile_active) : TileFlags{true, true, true};
   if (SPARSE && !flags.any()) {  // uniform: the gradient passes through
     if (grad_color) copy_tile(a, tp, grad_out, grad_color);
@@ -951,7 +953,7 @@ extern "C" int dr_antialias_forward(const DrAntialiasArgs* a, void* pairs, size_
   const int64_t blocks = tile_blocks(a->batch, a->height, a->width);
   aa_pairs_kernel<<<blocks, 256, 0, (hipStream_t)stream>>>(*a, t, bits, tiles);
   if (a->channels <= 0) return launch_status();
-  return channel_groups(a->channels, [&](auto nc) {
+  return exact_channels(a->channels, [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
     if (sparse)
       aa_blend_kernel<NC, true><<<blocks, 256, 0, (hipStream_t)stream>>>(*a, t, bits, tiles, out);
@@ -979,7 +981,7 @@ extern "C" int dr_antialias_backward(const DrAntialiasArgs* a, const void* pairs
   const bool sparse = sparse_pairs(a);
   if (!sparse) tiles = nullptr;
   const int64_t blocks = tile_blocks(a->batch, a->height, a->width);
-  return channel_groups(a->channels, [&](auto nc) {
+  return exact_channels(a->channels, [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
     if (sparse)
       aa_bwd_kernel<NC, true><<<blocks, 256, 0, (hipStream_t)stream>>>(

@@ -50,58 +50,30 @@ __device__ __forceinline__ void store4(float* p, float4 v) { *reinterpret_cast<f
 // Hardware fp32 atomic add (the buffers are ordinary coarse-grained device memory).
 __device__ __forceinline__ void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
 
-// N consecutive floats at p with the widest loads their alignment allows (16 bytes for N a
-// multiple of 4, 8 bytes for N = 2); false, with nothing loaded, when p is not so aligned. Gathers
-// of whole rows this way cost one memory instruction per 16 bytes instead of one per channel.
+// N consecutive floats at p, in one memory instruction for up to four of them. The copies state
+// no more than a float's alignment, which is all that this target's wide global loads and stores
+// need; a test of the address for a scalar path beside a wide one made the compiler split the
+// last access that the two have in common (texture forward at 8 x 1024^2, 4 channels: 127 -> 112 us).
 template <int N>
-__device__ __forceinline__ bool load_wide(const float* p, float (&v)[N]) {
-  if constexpr (N % 4 == 0) {
-    if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
-#pragma unroll
-    for (int i = 0; i < N / 4; ++i) {
-      const float4 q = reinterpret_cast<const float4*>(p)[i];
-      v[4 * i] = q.x;
-      v[4 * i + 1] = q.y;
-      v[4 * i + 2] = q.z;
-      v[4 * i + 3] = q.w;
-    }
-    return true;
-  } else if constexpr (N == 2) {
-    if (reinterpret_cast<uintptr_t>(p) & 7u) return false;
-    const float2 q = *reinterpret_cast<const float2*>(p);
-    v[0] = q.x;
-    v[1] = q.y;
-    return true;
-  }
-  return false;
+__device__ __forceinline__ void load_floats(const float* p, float (&v)[N]) {
+  __builtin_memcpy(v, p, sizeof(v));
 }
-
 template <int N>
-__device__ __forceinline__ bool store_wide(float* p, const float (&v)[N]) {
-  if constexpr (N % 4 == 0) {
-    if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
-#pragma unroll
-    for (int i = 0; i < N / 4; ++i)
-      reinterpret_cast<float4*>(p)[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    return true;
-  } else if constexpr (N == 2) {
-    if (reinterpret_cast<uintptr_t>(p) & 7u) return false;
-    *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
-    return true;
-  }
-  return false;
+__device__ __forceinline__ void store_floats(float* p, const float (&v)[N]) {
+  __builtin_memcpy(p, v, sizeof(v));
 }
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
-// Launches of kernels templated on NC channels per group: 1-4 as they are, more in groups of 4.
+// f(channels) with the channel count as a constant, 0 for more than four.
 template <typename F>
-int channel_groups(int channels, F f) {
+int exact_channels(int channels, F f) {
   switch (channels) {
     case 1: return f(std::integral_constant<int, 1>());
     case 2: return f(std::integral_constant<int, 2>());
     case 3: return f(std::integral_constant<int, 3>());
-    default: return f(std::integral_constant<int, 4>());
+    case 4: return f(std::integral_constant<int, 4>());
+    default: return f(std::integral_constant<int, 0>());
   }
 }
 

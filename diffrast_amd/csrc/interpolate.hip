@@ -54,41 +54,16 @@ __device__ __forceinline__ Pixel load_pixel(const DrInterpolateArgs& a, int64_t 
 template <int N, bool WHOLE = false>
 __device__ __forceinline__ void load_rows(const float* attr, const Pixel& p, int C, int c0,
                                           float (&A)[3][N]) {
-  // Whole-row loads when every row of the pass is 16-byte aligned: a condition on the buffer
-  // and the channel count alone, the same for every lane.
-  if constexpr (N % 4 == 0) {
-    if (C % 4 == 0 && c0 + N <= C && (reinterpret_cast<uintptr_t>(attr) & 15u) == 0) {
+  if (WHOLE || c0 + N <= C) {  // uniform
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const float4* row = reinterpret_cast<const float4*>(attr + (int64_t)p.row[k] * C + c0);
-#pragma unroll
-        for (int i = 0; i < N / 4; ++i) {
-          const float4 q = row[i];
-          A[k][4 * i] = q.x;
-          A[k][4 * i + 1] = q.y;
-          A[k][4 * i + 2] = q.z;
-          A[k][4 * i + 3] = q.w;
-        }
-      }
-      return;
-    }
-  }
-  if constexpr (N == 2) {
-    if (C == 2 && (reinterpret_cast<uintptr_t>(attr) & 7u) == 0) {
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const float2 q = reinterpret_cast<const float2*>(attr)[p.row[k]];
-        A[k][0] = q.x;
-        A[k][1] = q.y;
-      }
-      return;
-    }
+    for (int k = 0; k < 3; ++k) load_floats(attr + (int64_t)p.row[k] * C + c0, A[k]);
+    return;
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float* row = attr + (int64_t)p.row[k] * C + c0;
 #pragma unroll
-    for (int c = 0; c < N; ++c) A[k][c] = (WHOLE || c0 + c < C) ? row[c] : 0.0f;
+    for (int c = 0; c < N; ++c) A[k][c] = c0 + c < C ? row[c] : 0.0f;
   }
 }
 
@@ -160,8 +135,7 @@ __global__ __launch_bounds__(256) void interp_fwd_kernel(DrInterpolateArgs a,
       }
     }
     float* o = out + pixel[j] * NC;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) o[c] = res[c];
+    store_floats(o, res);
   }
 }
 
@@ -319,12 +293,15 @@ __global__ __launch_bounds__(256) void interp_bwd_kernel(DrInterpolateArgs a,
     float A[3][N], G[N];
     const bool live = p.valid;
     if (live) load_rows<N>(a.attr, p, C, c0, A);
-    const bool wide = live && c0 + N <= C && load_wide<N>(g + c0, G);
+    if (live && c0 + N <= C) {
+      load_floats(g + c0, G);
+    } else {
 #pragma unroll
-    for (int c = 0; c < N; ++c) {
-      if (!live) A[0][c] = A[1][c] = A[2][c] = 0.0f;
-      if (!wide) G[c] = (live && c0 + c < C) ? g[c0 + c] : 0.0f;
+      for (int c = 0; c < N; ++c) G[c] = (live && c0 + c < C) ? g[c0 + c] : 0.0f;
     }
+#pragma unroll
+    for (int c = 0; c < N; ++c)
+      if (!live) A[0][c] = A[1][c] = A[2][c] = 0.0f;
     // Vertex k, channel c at v[N k + c].
     float v[3 * N];
 #pragma unroll
@@ -448,10 +425,12 @@ __global__ __launch_bounds__(256) void interp_bwd_rast_kernel(DrInterpolateArgs 
     for (int j = 0; j < PPT; ++j) {
       const bool live = p[j].valid;
       const float* g = grad_out + (live ? pixel[j] * C : 0);
-      const bool wide = live && c0 + N <= C && load_wide<N>(g + c0, G[j]);
-      if (!wide)
+      if (live && c0 + N <= C) {
+        load_floats(g + c0, G[j]);
+      } else {
 #pragma unroll
         for (int c = 0; c < N; ++c) G[j][c] = (live && c0 + c < C) ? g[c0 + c] : 0.0f;
+      }
     }
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
@@ -582,9 +561,9 @@ extern "C" int dr_interpolate_forward(const DrInterpolateArgs* a, float* out, fl
       });
     });
   }
-  return channel_groups(args.channels, [&](auto nc) {  // 1-4
+  return exact_channels(args.channels, [&](auto nc) {
     return with_derivatives(args.num_diff > 0, [&](auto diff) {
-      constexpr int NC = decltype(nc)::value;
+      constexpr int NC = decltype(nc)::value > 0 ? decltype(nc)::value : 1;  // 1-4 here
       constexpr bool DIFF = decltype(diff)::value;
       constexpr int PPT = 2;  // pixels per thread
       constexpr int TW = kGatherTileWidth;

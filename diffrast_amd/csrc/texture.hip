@@ -25,31 +25,31 @@ namespace {
 
 using namespace tex;
 
+// Channels [c0, c0 + N) of a texel or pixel at p, 0 past C.
+template <int N>
+__device__ __forceinline__ void load_channels(const float* __restrict__ p, int C, int c0,
+                                              float (&v)[N]) {
+  if (c0 + N <= C) {  // uniform; known when compiling for 1-4 channels
+    load_floats(p + c0, v);
+    return;
+  }
+#pragma unroll
+  for (int c = 0; c < N; ++c) v[c] = c0 + c < C ? p[c0 + c] : 0.0f;
+}
+
 // Channels [c0, c0 + N) of the four taps (0 past C or for an invalid tap), all loads issued
 // together.
 template <int N>
 __device__ __forceinline__ void fetch_taps(const float* __restrict__ texels, const Bilinear<float>& L,
                                            int C, int c0, float (&t)[4][N]) {
-  if constexpr (N == 4) {
-    // Four-channel texels on a 16-byte aligned buffer: one 16-byte load per tap.
-    if (C == 4 && (reinterpret_cast<uintptr_t>(texels) & 15u) == 0) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const float4 v = L.valid[k] ? *reinterpret_cast<const float4*>(texels + (size_t)L.index[k] * 4)
-                                    : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        t[k][0] = v.x;
-        t[k][1] = v.y;
-        t[k][2] = v.z;
-        t[k][3] = v.w;
-      }
-      return;
-    }
-  }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float* row = texels + (size_t)L.index[k] * C + c0;
+    if (L.valid[k]) {
+      load_channels<N>(texels + (size_t)L.index[k] * C, C, c0, t[k]);
+    } else {
 #pragma unroll
-    for (int c = 0; c < N; ++c) t[k][c] = (L.valid[k] && c0 + c < C) ? row[c] : 0.0f;
+      for (int c = 0; c < N; ++c) t[k][c] = 0.0f;
+    }
   }
 }
 
@@ -59,14 +59,19 @@ __device__ __forceinline__ void tap_column(const float (&t)[4][N], int c, float 
   for (int k = 0; k < 4; ++k) out[k] = t[k][c];
 }
 
-// NC channels per pass (the channel count when it is 1-4; 4 with a loop for more). Every tap
-// of a pass is loaded before its stores. FILTER and BOUNDARY: a.filter and a.boundary, fixed
+// Channels per pass of a kernel for CHANNELS channels: 1-4 of them, or 0 for more, in fours.
+template <int CHANNELS>
+constexpr int kPassChannels = CHANNELS == 0 ? 4 : CHANNELS;
+
+// CHANNELS: the channel count when it is 1-4, 0 for more. Every tap of a pass is loaded before
+// its stores. FILTER and BOUNDARY: a.filter and a.boundary, fixed
 // when compiling (DR_BOUNDARY_CUBE for cube maps; FILTER may be kAnyMode: read at run time).
-template <int NC, bool CUBE, int FILTER, int BOUNDARY>
+template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
 __global__ __launch_bounds__(256) void tex_fwd_kernel(DrTextureArgs a, float* __restrict__ out) {
+  constexpr int NC = kPassChannels<CHANNELS>;
   const int64_t pixel = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (pixel >= (int64_t)a.batch * a.height * a.width) return;
-  const int C = a.channels;
+  const int C = CHANNELS > 0 ? CHANNELS : a.channels;
   float* o = out + pixel * C;
   Lookup<float> K;
   lookup_setup<float, CUBE, FILTER>(a, pixel, K);
@@ -109,11 +114,9 @@ __global__ __launch_bounds__(256) void tex_fwd_kernel(DrTextureArgs a, float* __
       }
       if (bad) res[c] = nan;
     }
-    if constexpr (NC == 4) {
-      if (C == 4 && (reinterpret_cast<uintptr_t>(o) & 15u) == 0) {
-        *reinterpret_cast<float4*>(o) = make_float4(res[0], res[1], res[2], res[3]);
-        continue;
-      }
+    if (c0 + NC <= C) {
+      store_floats(o + c0, res);
+      continue;
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c)
@@ -133,20 +136,7 @@ __device__ __forceinline__ void level_coordinate_grads(const Bilinear<float>& L,
   for (int c0 = 0; c0 < C; c0 += N) {
     float t[4][N], gc[N];
     fetch_taps<N>(texels, L, C, c0, t);
-    bool loaded = false;
-    if constexpr (N == 4) {
-      if (C == 4 && (reinterpret_cast<uintptr_t>(g) & 15u) == 0) {
-        const float4 v = *reinterpret_cast<const float4*>(g);
-        gc[0] = v.x;
-        gc[1] = v.y;
-        gc[2] = v.z;
-        gc[3] = v.w;
-        loaded = true;
-      }
-    }
-    if (!loaded)
-#pragma unroll
-      for (int c = 0; c < N; ++c) gc[c] = c0 + c < C ? g[c0 + c] : 0.0f;
+    load_channels<N>(g, C, c0, gc);
 #pragma unroll
     for (int c = 0; c < N; ++c) {
       if (c0 + c >= C) continue;
@@ -175,19 +165,21 @@ __device__ __forceinline__ void level_taps(const Bilinear<float>& L, float level
   }
 }
 
-// The 2D kernels are held to 72 VGPRs: seven waves per SIMD, as many as the table's LDS allows
-// (measured: 393 -> 388 us at 8 x 1024^2 with a 1024^2 texture, against six waves at 74 VGPRs;
-// the cube-map kernels spill at such budgets and keep their own).
-template <int NC, bool CUBE, int FILTER, int BOUNDARY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : 7))) void
+// The 2D kernels of up to 4 channels are held to 64 VGPRs: eight waves per SIMD, as many as the
+// table's LDS allows (355 -> 345 us at 8 x 1024^2 with a 1024^2 texture, against seven waves at
+// 65; with more channels seven are faster by 1 %; the cube-map kernels spill at such budgets,
+// 239 -> 320 us at seven waves, and keep their own).
+template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : (CHANNELS > 0 ? 8 : 7)))) void
 tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float* grad_uv,
                float* grad_uv_da, float* grad_bias) {
+  constexpr int NC = kPassChannels<CHANNELS>;
   using Table = RowTable<512, 4>;
   __shared__ Table table;
   table.init();
   const TilePixel tp = tile_pixel(a.batch, a.height, a.width);
   const int64_t pixel = tp.pixel;
-  const int C = a.channels;
+  const int C = CHANNELS > 0 ? CHANNELS : a.channels;
   constexpr bool cube = CUBE;
   const float* g = grad_out + (tp.inside ? pixel * C : 0);
   const int64_t tex_off = a.tex_batch > 1 ? (int64_t)tp.b * a.num_texels : 0;
@@ -277,10 +269,8 @@ tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float
     if (tap_key[k] != Table::kEmpty) w_max = fmaxf(w_max, fabsf(tap_weight[k]));
   for (int c0 = 0; c0 < C; c0 += 4) {
     const int n = min(4, C - c0);
-    float gc[4] = {0.f, 0.f, 0.f, 0.f};
-    if (!(n == 4 && load_wide<4>(g + c0, gc)))
-#pragma unroll
-      for (int c = 0; c < 4; ++c) gc[c] = c < n ? g[c0 + c] : 0.0f;
+    float gc[4];
+    load_channels<4>(g, C, c0, gc);
     // The largest |g[c] * weight[k]| of this lane (rounding is monotone, so the product of the
     // two largest factors is the largest product).
     float g_max = 0.0f;
@@ -736,7 +726,7 @@ MipLevels copy_levels(int n, const int32_t* h, const int32_t* w, const int64_t* 
   return L;
 }
 
-// Calls f(channel group, cube, filter, boundary) with each as a compile-time constant
+// Calls f(channels (0: more than 4), cube, filter, boundary) with each as a compile-time constant
 // (std::integral_constant), from a's channel count and modes (checked by valid_args): the
 // kernels are compiled for every combination, each without the other modes' code.
 template <typename F>
@@ -754,7 +744,7 @@ int texture_modes(const DrTextureArgs& a, F f) {
         return f(nc, std::false_type(), filter, integral_constant<int, DR_BOUNDARY_ZERO>());
     }
   };
-  return channel_groups(a.channels, [&](auto nc) {
+  auto with_filter = [&](auto nc) {
     using std::integral_constant;
     switch (a.filter) {
       case DR_FILTER_NEAREST:
@@ -766,7 +756,8 @@ int texture_modes(const DrTextureArgs& a, F f) {
       default:
         return with_boundary(nc, integral_constant<int, DR_FILTER_MIP_LINEAR>());
     }
-  });
+  };
+  return exact_channels(a.channels, with_filter);
 }
 
 bool valid_args(const DrTextureArgs* a) {

@@ -63,40 +63,49 @@ template <class S> constexpr S kLn2 = S(0.693147180559945309417232121458176568);
 
 // ---- cube geometry (_cube.py) -------------------------------------------------------------------
 
-// Per face: major axis, s axis and t axis as integer 3-vectors (_cube.py:31-33).
-__constant__ int kMajor[6][3] = {{1, 0, 0}, {-1, 0, 0}, {0, 1, 0}, {0, -1, 0}, {0, 0, 1}, {0, 0, -1}};
-__constant__ int kSAxis[6][3] = {{0, 0, -1}, {0, 0, 1}, {1, 0, 0}, {1, 0, 0}, {1, 0, 0}, {-1, 0, 0}};
-__constant__ int kTAxis[6][3] = {{0, -1, 0}, {0, -1, 0}, {0, 0, 1}, {0, 0, -1}, {0, -1, 0}, {0, -1, 0}};
+// Faces are +x, -x, +y, -y, +z, -z, each with a major, an s and a t axis (_cube.py:31-33):
+//   major   x -x  y -y  z -z     s  -z  z  x  x  x -x     t  -y -y  z -z -y -y
 
-__device__ __forceinline__ int floor_div2(int v) { return v >= 0 ? v / 2 : -((-v + 1) / 2); }
+// v along a face's s axis, t axis and major axis: each is plus or minus one component, taken
+// with selects (table lookups would be divergent loads, and dot products of which two terms are
+// zero). v is finite: the zero terms would add nothing.
+template <class S>
+__device__ __forceinline__ S along_s(int face, S x, S z) {
+  const S v = face < 2 ? z : x;
+  return face == 0 || face == 5 ? -v : v;
+}
+template <class S>
+__device__ __forceinline__ S along_t(int face, S y, S z) {
+  const S v = (face >> 1) == 1 ? z : y;
+  return face == 2 ? v : -v;
+}
+template <class S>
+__device__ __forceinline__ S along_major(int face, S x, S y, S z) {
+  const S v = face < 2 ? x : (face < 4 ? y : z);
+  return (face & 1) != 0 ? -v : v;
+}
 
 // Fold a texel one step outside its face onto the neighbouring face (_cube.py:105-143).
 // Returns false beyond a corner, where no texel exists.
 __device__ __forceinline__ bool cube_fold(int& face, int& row, int& col, int size) {
   const bool over_col = col < 0 || col >= size;
   const bool over_row = row < 0 || row >= size;
-  const int sc = 2 * col + 1 - size, tc = 2 * row + 1 - size;
-  int point[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    int p = size * kMajor[face][k] + sc * kSAxis[face][k] + tc * kTAxis[face][k];
-    p = min(max(p, -size), size);
-    if (over_col || over_row) p -= kMajor[face][k];
-    point[k] = p;
-  }
-  int axis = 0;
-  int best = abs(point[0]);
-  if (abs(point[1]) > best) { axis = 1; best = abs(point[1]); }
-  if (abs(point[2]) > best) axis = 2;
-  face = 2 * axis + (point[axis] < 0 ? 1 : 0);
-  int s_dot = 0, t_dot = 0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    s_dot += point[k] * kSAxis[face][k];
-    t_dot += point[k] * kTAxis[face][k];
-  }
-  col = max(floor_div2(s_dot + size - 1), 0);
-  row = max(floor_div2(t_dot + size - 1), 0);
+  const int axis = face >> 1, sign = (face & 1) != 0 ? -1 : 1;
+  // The texel's centre in half texels, clamped onto the cube, one step back along the old major
+  // axis where it lay past an edge.
+  const int sc = min(max(2 * col + 1 - size, -size), size);
+  const int tc = min(max(2 * row + 1 - size, -size), size);
+  const int major = sign * (size - (over_col || over_row ? 1 : 0));
+  const int x = axis == 0 ? major : (axis == 1 || sign > 0 ? sc : -sc);
+  const int y = axis == 1 ? major : -tc;
+  const int z = axis == 2 ? major : (axis == 1 ? sign * tc : -sign * sc);
+  // The face it lies on now: the first axis of the largest magnitude.
+  const int ax = abs(x), ay = abs(y), az = abs(z);
+  const int to = az > max(ax, ay) ? 2 : (ay > ax ? 1 : 0);
+  const int along = to == 0 ? x : (to == 1 ? y : z);
+  face = 2 * to + (along < 0 ? 1 : 0);
+  col = max((along_s(face, x, z) + size - 1) >> 1, 0);
+  row = max((along_t(face, y, z) + size - 1) >> 1, 0);
   return !(over_col && over_row);
 }
 
@@ -104,7 +113,7 @@ template <class S>
 struct CubeProj {
   bool valid, undefined;
   int face;
-  S length, ma, rs, rt;
+  S length, rs, rt;
   S dn[3];
   S da[3][2];           // clamped, scaled derivatives
   bool da_pass[3][2];   // inside the clamp
@@ -113,7 +122,9 @@ struct CubeProj {
   S st_da[4];           // ds/dx, ds/dy, dt/dx, dt/dy
 };
 
-// Face selection and face coordinates of a direction (_cube.py:44-102).
+// Face selection and face coordinates of a direction (_cube.py:44-102). The direction scaled by
+// its largest component has exactly 1 along the major axis (x / |x|), so the divisions by that
+// component leave every value as it is and are left out.
 template <class S>
 __device__ __forceinline__ void cube_project(const S* dir, const S* dir_da, CubeProj<S>& P) {
   S d[3] = {dir[0], dir[1], dir[2]};
@@ -133,14 +144,8 @@ __device__ __forceinline__ void cube_project(const S* dir, const S* dir_da, Cube
   P.length = s_max(s_max(ax, ay), az);
 #pragma unroll
   for (int k = 0; k < 3; ++k) P.dn[k] = d[k] / P.length;
-  const int* M = kMajor[P.face];
-  const int* A = kSAxis[P.face];
-  const int* T = kTAxis[P.face];
-  P.ma = P.dn[0] * (S)M[0] + P.dn[1] * (S)M[1] + P.dn[2] * (S)M[2];
-  const S sc = P.dn[0] * (S)A[0] + P.dn[1] * (S)A[1] + P.dn[2] * (S)A[2];
-  const S tc = P.dn[0] * (S)T[0] + P.dn[1] * (S)T[1] + P.dn[2] * (S)T[2];
-  P.rs = sc / P.ma;
-  P.rt = tc / P.ma;
+  P.rs = along_s(P.face, P.dn[0], P.dn[2]);
+  P.rt = along_t(P.face, P.dn[1], P.dn[2]);
   P.st[0] = S(0.5) * (P.rs + S(1));
   P.st[1] = S(0.5) * (P.rt + S(1));
   P.undefined = false;
@@ -159,15 +164,15 @@ __device__ __forceinline__ void cube_project(const S* dir, const S* dir_da, Cube
     }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    P.d_ma[j] = P.da[0][j] * (S)M[0] + P.da[1][j] * (S)M[1] + P.da[2][j] * (S)M[2];
-    P.d_sc[j] = P.da[0][j] * (S)A[0] + P.da[1][j] * (S)A[1] + P.da[2][j] * (S)A[2];
-    P.d_tc[j] = P.da[0][j] * (S)T[0] + P.da[1][j] * (S)T[1] + P.da[2][j] * (S)T[2];
+    P.d_ma[j] = along_major(P.face, P.da[0][j], P.da[1][j], P.da[2][j]);
+    P.d_sc[j] = along_s(P.face, P.da[0][j], P.da[2][j]);
+    P.d_tc[j] = along_t(P.face, P.da[1][j], P.da[2][j]);
   }
   const S nan = s_nan<S>();
-  P.st_da[0] = P.undefined ? nan : S(0.5) * (P.d_sc[0] - P.rs * P.d_ma[0]) / P.ma;
-  P.st_da[1] = P.undefined ? nan : S(0.5) * (P.d_sc[1] - P.rs * P.d_ma[1]) / P.ma;
-  P.st_da[2] = P.undefined ? nan : S(0.5) * (P.d_tc[0] - P.rt * P.d_ma[0]) / P.ma;
-  P.st_da[3] = P.undefined ? nan : S(0.5) * (P.d_tc[1] - P.rt * P.d_ma[1]) / P.ma;
+  P.st_da[0] = P.undefined ? nan : S(0.5) * (P.d_sc[0] - P.rs * P.d_ma[0]);
+  P.st_da[1] = P.undefined ? nan : S(0.5) * (P.d_sc[1] - P.rs * P.d_ma[1]);
+  P.st_da[2] = P.undefined ? nan : S(0.5) * (P.d_tc[0] - P.rt * P.d_ma[0]);
+  P.st_da[3] = P.undefined ? nan : S(0.5) * (P.d_tc[1] - P.rt * P.d_ma[1]);
 }
 
 // Gradient of cube_project: from d(loss)/d(st) and d(loss)/d(st_da) to the direction and
@@ -176,12 +181,15 @@ template <class S>
 __device__ __forceinline__ void cube_project_backward(const CubeProj<S>& P, S g_s, S g_t,
                                                       bool use_sda, const S (&g_sda)[4],
                                                       S (&grad_dir)[3], S (&grad_dir_da)[6]) {
-  const int* M = kMajor[P.face];
-  const int* A = kSAxis[P.face];
-  const int* T = kTAxis[P.face];
-  // Gradient only: multiplies by the reciprocals (two divisions instead of 25; each product
+  // The axes as coefficients, by selects (see cube_project).
+  const int axis = P.face >> 1;
+  const S sign = (P.face & 1) != 0 ? S(-1) : S(1);
+  const S M[3] = {axis == 0 ? sign : S(0), axis == 1 ? sign : S(0), axis == 2 ? sign : S(0)};
+  const S A[3] = {axis == 0 ? S(0) : (axis == 1 ? S(1) : sign), S(0), axis == 0 ? -sign : S(0)};
+  const S T[3] = {S(0), axis == 1 ? S(0) : S(-1), axis == 1 ? sign : S(0)};
+  // Gradient only: multiplies by the reciprocal (one division instead of nine; each product
   // is within two ulp of the quotient).
-  const S inv_ma = S(1) / P.ma, inv_length = S(1) / P.length;
+  const S inv_length = S(1) / P.length;
   S g_rs = S(0.5) * g_s, g_rt = S(0.5) * g_t, g_ma = S(0);
   S g_dsc[2] = {S(0), S(0)}, g_dtc[2] = {S(0), S(0)}, g_dma[2] = {S(0), S(0)};
   if (use_sda && !P.undefined) {
@@ -189,26 +197,26 @@ __device__ __forceinline__ void cube_project_backward(const CubeProj<S>& P, S g_
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const S ds = P.st_da[j], dt = P.st_da[2 + j];
-      g_rs += gds[j] * (S(-0.5) * P.d_ma[j] * inv_ma);
-      g_rt += gdt[j] * (S(-0.5) * P.d_ma[j] * inv_ma);
-      g_ma -= (gds[j] * ds + gdt[j] * dt) * inv_ma;
-      g_dsc[j] = S(0.5) * gds[j] * inv_ma;
-      g_dtc[j] = S(0.5) * gdt[j] * inv_ma;
-      g_dma[j] = S(-0.5) * (gds[j] * P.rs + gdt[j] * P.rt) * inv_ma;
+      g_rs += gds[j] * (S(-0.5) * P.d_ma[j]);
+      g_rt += gdt[j] * (S(-0.5) * P.d_ma[j]);
+      g_ma -= (gds[j] * ds + gdt[j] * dt);
+      g_dsc[j] = S(0.5) * gds[j];
+      g_dtc[j] = S(0.5) * gdt[j];
+      g_dma[j] = S(-0.5) * (gds[j] * P.rs + gdt[j] * P.rt);
     }
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      S g = g_dsc[j] * (S)A[k] + g_dtc[j] * (S)T[k] + g_dma[j] * (S)M[k];
+      S g = g_dsc[j] * A[k] + g_dtc[j] * T[k] + g_dma[j] * M[k];
       g = (P.valid && !P.undefined && P.da_pass[k][j]) ? g * inv_length : S(0);
       grad_dir_da[2 * k + j] = g;
     }
-  g_ma -= (g_rs * P.rs + g_rt * P.rt) * inv_ma;
+  g_ma -= (g_rs * P.rs + g_rt * P.rt);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const S g_dn = (g_rs * (S)A[k] + g_rt * (S)T[k]) * inv_ma + g_ma * (S)M[k];
+    const S g_dn = (g_rs * A[k] + g_rt * T[k]) + g_ma * M[k];
     grad_dir[k] = P.valid ? g_dn * inv_length : S(0);
   }
 }
@@ -309,6 +317,7 @@ struct Bilinear {
   // Cube corners: taps beyond two edges count as the mean of the other three.
   bool cube;
   S corner[4];  // 1 where (left|right) & (above|below) for taps 00, 01, 10, 11
+  bool at_corner;  // any of them is
 };
 
 // CUBE: boundary is DR_BOUNDARY_CUBE, else one of the 2D boundaries (known when compiling, so
@@ -329,7 +338,17 @@ __device__ __forceinline__ Bilinear<S> bilinear_setup(S s, S t, int face, int h,
   L.size_y = (S)h;
   const int col = (int)x0, row = (int)y0;
   L.cube = CUBE;
-  if constexpr (CUBE) {
+  const bool inside = row >= 0 && row + 1 < h && col >= 0 && col + 1 < w;
+  if (CUBE && inside) {
+    // All four taps on the face: nothing to fold.
+    const uint32_t first = (uint32_t)offset + (uint32_t)(face * h + row) * (uint32_t)w + (uint32_t)col;
+    L.index[0] = first;
+    L.index[1] = first + 1u;
+    L.index[2] = first + (uint32_t)w;
+    L.index[3] = first + (uint32_t)w + 1u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) L.valid[k] = true;
+  } else if constexpr (CUBE) {
     L.valid[0] = tap(row, col, face, h, w, offset, boundary, L.index[0]);
     L.valid[1] = tap(row, col + 1, face, h, w, offset, boundary, L.index[1]);
     L.valid[2] = tap(row + 1, col, face, h, w, offset, boundary, L.index[2]);
@@ -348,12 +367,14 @@ __device__ __forceinline__ Bilinear<S> bilinear_setup(S s, S t, int face, int h,
     L.valid[2] = R.valid[1] && K.valid[0];
     L.valid[3] = R.valid[1] && K.valid[1];
   }
+  L.at_corner = false;
   if (L.cube) {
     const bool left = col < 0, right = col + 1 >= w, above = row < 0, below = row + 1 >= h;
     L.corner[0] = (left && above) ? S(1) : S(0);
     L.corner[1] = (right && above) ? S(1) : S(0);
     L.corner[2] = (left && below) ? S(1) : S(0);
     L.corner[3] = (right && below) ? S(1) : S(0);
+    L.at_corner = (left || right) && (above || below);
   }
   return L;
 }
@@ -366,7 +387,11 @@ __device__ __forceinline__ S bilinear_value(const Bilinear<S>& L, const S (&t)[4
   if (L.cube) {
     const S missing = (S(1) - fy) * ((S(1) - fx) * L.corner[0] + fx * L.corner[1]) +
                       fy * ((S(1) - fx) * L.corner[2] + fx * L.corner[3]);
-    out = out + missing * (t[0] + t[1] + t[2] + t[3]) / S(3);
+    // Away from the corners missing is 0 and the third of the product is the product (0, or
+    // NaN where a tap is not finite).
+    S share = missing * (t[0] + t[1] + t[2] + t[3]);
+    if (L.at_corner) share = share / S(3);
+    out = out + share;
   }
   return out;
 }

@@ -59,19 +59,12 @@ __device__ __forceinline__ void tap_column(const float (&t)[4][N], int c, float 
   for (int k = 0; k < 4; ++k) out[k] = t[k][c];
 }
 
-// Channels per pass of a kernel for CHANNELS channels: 1-4 of them, or 0 for more, in fours.
-template <int CHANNELS>
-constexpr int kPassChannels = CHANNELS == 0 ? 4 : CHANNELS;
-
-// CHANNELS: the channel count when it is 1-4, 0 for more. Every tap of a pass is loaded before
-// its stores. FILTER and BOUNDARY: a.filter and a.boundary, fixed
-// when compiling (DR_BOUNDARY_CUBE for cube maps; FILTER may be kAnyMode: read at run time).
-template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
+// One to four channels. Every tap is loaded before the stores. FILTER and BOUNDARY: a.filter and
+// a.boundary, fixed when compiling (DR_BOUNDARY_CUBE for cube maps).
+template <int C, bool CUBE, int FILTER, int BOUNDARY>
 __global__ __launch_bounds__(256) void tex_fwd_kernel(DrTextureArgs a, float* __restrict__ out) {
-  constexpr int NC = kPassChannels<CHANNELS>;
   const int64_t pixel = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (pixel >= (int64_t)a.batch * a.height * a.width) return;
-  const int C = CHANNELS > 0 ? CHANNELS : a.channels;
   float* o = out + pixel * C;
   Lookup<float> K;
   lookup_setup<float, CUBE, FILTER>(a, pixel, K);
@@ -97,30 +90,166 @@ __global__ __launch_bounds__(256) void tex_fwd_kernel(DrTextureArgs a, float* __
   const Bilinear<float> L1 = two ? level_setup<CUBE, BOUNDARY>(a, K, D, 1) : L0;
   const bool bad = K.bad || L0.bad || (two && L1.bad);
   const float frac = K.level_weight[1];
-  for (int c0 = 0; c0 < C; c0 += NC) {
-    float t[4][NC], u[4][NC];
-    fetch_taps<NC>(texels, L0, C, c0, t);
-    if (two) fetch_taps<NC>(texels, L1, C, c0, u);
-    float res[NC];
+  float t[4][C], u[4][C], res[C];
+  fetch_taps<C>(texels, L0, C, 0, t);
+  if (two) fetch_taps<C>(texels, L1, C, 0, u);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      float tc[4], uc[4];
-      tap_column(t, c, tc);
-      if (two) {
-        tap_column(u, c, uc);
-        res[c] = bilinear_value(L0, tc) * (1.0f - frac) + bilinear_value(L1, uc) * frac;
-      } else {
-        res[c] = bilinear_value(L0, tc);
+  for (int c = 0; c < C; ++c) {
+    float tc[4], uc[4];
+    tap_column(t, c, tc);
+    if (two) {
+      tap_column(u, c, uc);
+      res[c] = bilinear_value(L0, tc) * (1.0f - frac) + bilinear_value(L1, uc) * frac;
+    } else {
+      res[c] = bilinear_value(L0, tc);
+    }
+    if (bad) res[c] = nan;
+  }
+  store_floats(o, res);
+}
+
+// A pixel's lookup as the wide kernel keeps it in LDS: per level its taps (kNoTexel: reads zero)
+// and fractions, the weight of the missing tap at a cube corner, the share of the second level,
+// the image, and how many levels (0: nearest, one tap; kBadLookup: NaN).
+constexpr uint32_t kNoTexel = 0xffffffffu;
+constexpr int kBadLookup = -1;
+template <bool CUBE>
+struct WideLevel {
+  uint32_t index[4];
+  float fx, fy;
+  float missing;  // the same taps' mean counts this much (a third of their sum: at_corner)
+  bool at_corner;
+};
+template <>
+struct WideLevel<false> {
+  uint32_t index[4];
+  float fx, fy;
+};
+template <bool CUBE>
+struct WideLookup {
+  WideLevel<CUBE> level[2];
+  float frac;
+  int levels;
+  uint32_t image;
+};
+
+template <bool CUBE>
+__device__ __forceinline__ void keep_level(const Bilinear<float>& L, WideLevel<CUBE>& W) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) W.index[k] = L.valid[k] ? L.index[k] : kNoTexel;
+  W.fx = L.fx;
+  W.fy = L.fy;
+  if constexpr (CUBE) {
+    W.missing = (1.0f - L.fy) * ((1.0f - L.fx) * L.corner[0] + L.fx * L.corner[1]) +
+                L.fy * ((1.0f - L.fx) * L.corner[2] + L.fx * L.corner[3]);
+    W.at_corner = L.at_corner;
+  }
+}
+
+// N channels of a level's lookup, from texels + element offset (bilinear_value's arithmetic).
+template <int N, bool CUBE>
+__device__ __forceinline__ void wide_value(const WideLevel<CUBE>& W, const float (&t)[4][N],
+                                           float (&v)[N]) {
+  const float fx = W.fx, fy = W.fy;
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    v[c] = (1.0f - fy) * ((1.0f - fx) * t[0][c] + fx * t[1][c]) +
+           fy * ((1.0f - fx) * t[2][c] + fx * t[3][c]);
+    if constexpr (CUBE) {
+      float share = W.missing * (t[0][c] + t[1][c] + t[2][c] + t[3][c]);
+      if (W.at_corner) share = share / 3.0f;
+      v[c] = v[c] + share;
+    }
+  }
+}
+
+// More than four channels, N of them (4, 2 or 1: a divisor of the count) to a lane: each thread
+// works out one pixel's taps, then consecutive lanes take a pixel's channels in turn, so that
+// texels and output go in whole lines and the taps are worked out once. (A pixel per thread and
+// four channels at a time, two 720 x 1280 images with 16 channels: 180 us; this one 60.)
+template <int N, bool CUBE, int FILTER, int BOUNDARY>
+__global__ __launch_bounds__(256) void tex_fwd_wide_kernel(DrTextureArgs a,
+                                                           float* __restrict__ out) {
+  __shared__ WideLookup<CUBE> s_lookup[256];
+  const int64_t pixels = (int64_t)a.batch * a.height * a.width;
+  const int64_t pixel0 = (int64_t)blockIdx.x * 256, pixel = pixel0 + threadIdx.x;
+  if (pixel < pixels) {
+    WideLookup<CUBE>& W = s_lookup[threadIdx.x];
+    Lookup<float> K;
+    lookup_setup<float, CUBE, FILTER>(a, pixel, K);
+    W.image = a.tex_batch > 1 ? (uint32_t)(pixel / ((int64_t)a.height * a.width)) : 0u;
+    W.frac = 0.0f;
+    W.levels = K.levels;
+    if (K.dir_invalid) {  // reads zero
+      W.levels = 0;
+      W.level[0].index[0] = kNoTexel;
+    } else if (K.levels == 0) {
+      uint32_t index;
+      bool valid;
+      if (nearest_setup<BOUNDARY>(a, K, index, valid)) W.levels = kBadLookup;
+      W.level[0].index[0] = valid ? index : kNoTexel;
+    } else {
+      const LevelDims D = lookup_levels(a, K);
+      const Bilinear<float> L0 = level_setup<CUBE, BOUNDARY>(a, K, D, 0);
+      bool bad = K.bad || L0.bad;
+      keep_level(L0, W.level[0]);
+      if (K.levels == 2) {
+        const Bilinear<float> L1 = level_setup<CUBE, BOUNDARY>(a, K, D, 1);
+        bad = bad || L1.bad;
+        keep_level(L1, W.level[1]);
+        W.frac = K.level_weight[1];
       }
-      if (bad) res[c] = nan;
+      if (bad) W.levels = kBadLookup;
     }
-    if (c0 + NC <= C) {
-      store_floats(o + c0, res);
-      continue;
-    }
+  }
+  __syncthreads();
+  const int C = a.channels, per = C / N;  // elements per pixel
+  const int count = (int)min((int64_t)256, pixels - pixel0);
+  // A step of 256 elements moves (pixel, element) by (dj, de).
+  const int dj = 256 / per, de = 256 % per;
+  int j = (int)threadIdx.x / per, e = (int)threadIdx.x % per;
+  for (; j < count;) {
+    const WideLookup<CUBE>& W = s_lookup[j];
+    const float* texels = a.texels + (int64_t)W.image * a.num_texels * C + e * N;
+    auto fetch = [&](uint32_t index, float(&v)[N]) {
+      if (index != kNoTexel) {
+        load_floats(texels + (size_t)index * C, v);
+      } else {
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-      if (c0 + c < C) o[c0 + c] = res[c];
+        for (int c = 0; c < N; ++c) v[c] = 0.0f;
+      }
+    };
+    float res[N];
+    if (W.levels <= 0) {
+      if (W.levels == 0) {
+        fetch(W.level[0].index[0], res);
+      } else {
+#pragma unroll
+        for (int c = 0; c < N; ++c) res[c] = __int_as_float(0x7fc00000);
+      }
+    } else {
+      float t[4][N], u[4][N];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) fetch(W.level[0].index[k], t[k]);
+      if (W.levels == 2)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) fetch(W.level[1].index[k], u[k]);
+      wide_value(W.level[0], t, res);
+      if (W.levels == 2) {
+        const float frac = W.frac;
+        float above[N];
+        wide_value(W.level[1], u, above);
+#pragma unroll
+        for (int c = 0; c < N; ++c) res[c] = res[c] * (1.0f - frac) + above[c] * frac;
+      }
+    }
+    store_floats(out + (pixel0 + j) * C + e * N, res);
+    j += dj;
+    e += de;
+    if (e >= per) {
+      e -= per;
+      ++j;
+    }
   }
 }
 
@@ -169,6 +298,11 @@ __device__ __forceinline__ void level_taps(const Bilinear<float>& L, float level
 // table's LDS allows (355 -> 345 us at 8 x 1024^2 with a 1024^2 texture, against seven waves at
 // 65; with more channels seven are faster by 1 %; the cube-map kernels spill at such budgets,
 // 239 -> 320 us at seven waves, and keep their own).
+// Channels per pass of the backward kernel for CHANNELS channels: 1-4 of them, or 0 for more, in
+// fours.
+template <int CHANNELS>
+constexpr int kPassChannels = CHANNELS == 0 ? 4 : CHANNELS;
+
 template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : (CHANNELS > 0 ? 8 : 7)))) void
 tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float* grad_uv,
@@ -785,9 +919,19 @@ extern "C" int dr_texture_forward(const DrTextureArgs* a, float* out, void* stre
   if (pixels == 0) return DR_OK;
   const DrTextureArgs args = *a;
   return texture_modes(args, [&](auto nc, auto cube, auto filter, auto boundary) {
-    tex_fwd_kernel<decltype(nc)::value, decltype(cube)::value, decltype(filter)::value,
-                   decltype(boundary)::value>
-        <<<blocks_for(pixels, 256), 256, 0, (hipStream_t)stream>>>(args, out);
+    constexpr int NC = decltype(nc)::value, FILTER = decltype(filter)::value;
+    constexpr int BOUNDARY = decltype(boundary)::value;
+    constexpr bool CUBE = decltype(cube)::value;
+    const int blocks = blocks_for(pixels, 256);
+    const hipStream_t st = (hipStream_t)stream;
+    if constexpr (NC > 0)
+      tex_fwd_kernel<NC, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
+    else if (args.channels % 4 == 0)
+      tex_fwd_wide_kernel<4, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
+    else if (args.channels % 2 == 0)
+      tex_fwd_wide_kernel<2, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
+    else
+      tex_fwd_wide_kernel<1, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
     return launch_status();
   });
 }

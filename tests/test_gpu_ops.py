@@ -289,6 +289,39 @@ def test_texture_gradients_where_pixels_share_texels(filter_mode, pattern):
     assert_grads_close(grads[:1], grads[1:])
 
 
+@pytest.mark.parametrize("channels", [5, 6, 8, 20, 300])
+@pytest.mark.parametrize("boundary", [*BOUNDARIES, "cube"])
+@pytest.mark.parametrize("tex_batch", [1, 2])
+def test_texture_many_channels(channels, boundary, tex_batch):
+    # More than four channels go one, two or four to a lane, 300 of them past a workgroup's
+    # lanes; lookups that read nothing (NaN coordinates and levels, a zero direction), cube
+    # edges and corners, every filter; 2 x 20 x 24 pixels end in a partial workgroup.
+    gen = torch.Generator().manual_seed(channels)
+    cube = boundary == "cube"
+    tex = torch.randn(tex_batch, *((6, 16, 16) if cube else (13, 18)), channels, generator=gen)
+    if cube:
+        uv = torch.randint(-3, 4, (2, 20, 24, 3), generator=gen) / 3.0  # many exactly on edges
+        uv[1] += torch.randn(20, 24, 3, generator=gen)
+        uv_da = torch.randn(2, 20, 24, 6, generator=gen) * 0.2
+        uv[0, 0, 0] = 0.0
+    else:
+        _, uv, uv_da = tex_scene(seed=channels)
+    uv[0, 1, 1, 0] = float("nan")
+    uv_da[0, 2, 2, 1] = float("nan")
+    weights = torch.randn(2, 20, 24, channels, generator=gen)
+    for filter_mode in FILTERS:
+        da = uv_da if "mipmap" in filter_mode else None
+
+        def run(fn):
+            return lambda t, c, d: fn(t, c, d, filter_mode, boundary, None)
+
+        outs, grads = grads_of(run(hip.texture), [tex, uv, da], [weights], "cuda")
+        e_outs, e_grads = grads_of(run(R.texture), [tex, uv, da], [weights], "cpu")
+        assert torch.equal(outs[0].isnan(), e_outs[0].isnan()), filter_mode
+        assert rel_error(outs[0].nan_to_num(), e_outs[0].nan_to_num()) < VALUE_TOL, filter_mode
+        assert_grads_close(grads[:1], e_grads[:1])
+
+
 @pytest.mark.parametrize("max_mip_level", [0, 2])
 def test_texture_max_mip_level(max_mip_level):
     tex, uv, uv_da = tex_scene()

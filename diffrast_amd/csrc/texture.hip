@@ -294,17 +294,129 @@ __device__ __forceinline__ void level_taps(const Bilinear<float>& L, float level
   }
 }
 
-// The 2D kernels of up to 4 channels are held to 64 VGPRs: eight waves per SIMD, as many as the
-// table's LDS allows (355 -> 345 us at 8 x 1024^2 with a 1024^2 texture, against seven waves at
-// 65; with more channels seven are faster by 1 %; the cube-map kernels spill at such budgets,
-// 239 -> 320 us at seven waves, and keep their own).
+// What a pixel's 2D lookup depends on, as bits: coordinates, derivatives and bias.
+template <bool MIP>
+struct RawLookup {
+  uint32_t v[MIP ? 7 : 2];
+};
+
+template <bool MIP>
+__device__ __forceinline__ RawLookup<MIP> raw_lookup(const DrTextureArgs& a, int64_t pixel) {
+  RawLookup<MIP> r;
+  __builtin_memcpy(r.v, a.uv + 2 * pixel, 8);
+  if constexpr (MIP) {
+#pragma unroll
+    for (int i = 2; i < 7; ++i) r.v[i] = 0u;
+    if (a.uv_da) __builtin_memcpy(r.v + 2, a.uv_da + 4 * pixel, 16);
+    if (a.bias) __builtin_memcpy(r.v + 6, a.bias + pixel, 4);
+  }
+  return r;
+}
+
+// Texel gradients of strips (a wave's 16 x 4 pixels of a tile) whose pixels all share one lookup:
+// in practice the background, whose coordinates are zero. Its taps are the same texels
+// everywhere, and one texel takes atomic additions from all those tiles one after another (~9 ns
+// each), so of up to kStripTiles tiles side by side the first whose strip shares the lookup
+// takes the upstream gradients of the others' strips too. A wave finds out for itself:
+//   - the wave's taps differ: nothing changes (a register comparison is all it cost);
+//   - they are shared, by a strip further left too: the wave has nothing to add, its keys go;
+//   - they are shared, first here: lane k keeps tap k alone, and the result is the mask of the
+//     tiles, from this one on, whose gradients the wave sums (strip_sum).
+// Texture forward and backward with four tiles side by side, against none: a 1080 x 1920 image,
+// 79 % background, 3 channels 164 -> 131 us; two 720 x 1280 with 16 channels 564 -> 474; eight
+// 1024^2, 38 % background, 4 channels 495 -> 493, 79 % of one texel lookup each 477 -> 292. Eight
+// tiles are 1-8 % slower (a wave of the background looks at all of them), two up to 12 %.
+// Bit d of the result: the strip of the d-th tile to the right; 0: an ordinary wave.
+constexpr int kStripTiles = 4;
+
+template <bool MIP>
+__device__ __forceinline__ uint32_t shared_strips(const DrTextureArgs& a, const TilePixel& tp,
+                                                  uint32_t (&key)[8], float (&weight)[8]) {
+  // The first lane's pixel is inside the image unless the whole strip lies below it.
+  bool same = true;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    same = same && key[k] == (uint32_t)__builtin_amdgcn_readfirstlane((int)key[k]);
+    same = same && __float_as_int(weight[k]) ==
+                       __builtin_amdgcn_readfirstlane(__float_as_int(weight[k]));
+  }
+  if (__ballot(tp.inside && !same) != 0) return 0u;
+  if (__builtin_amdgcn_readfirstlane(tp.inside ? 1 : 0) == 0) return 0u;
+  const RawLookup<MIP> own = raw_lookup<MIP>(a, tp.inside ? tp.pixel : 0);
+  RawLookup<MIP> shared;
+#pragma unroll
+  for (int i = 0; i < (MIP ? 7 : 2); ++i)
+    shared.v[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)own.v[i]);
+  auto differs = [&](const RawLookup<MIP>& r) {
+    bool d = false;
+#pragma unroll
+    for (int i = 0; i < (MIP ? 7 : 2); ++i) d = d || r.v[i] != shared.v[i];
+    return d;
+  };
+  if (__ballot(tp.inside && differs(own)) != 0) return 0u;
+  const int at = __builtin_amdgcn_readfirstlane(tp.x / 16) % kStripTiles;
+  uint32_t found = 1u << at;
+#pragma unroll 2
+  for (int d = 0; d < kStripTiles; ++d) {
+    if (d == at) continue;  // uniform
+    const int x = tp.x + 16 * (d - at);
+    const int x0 = __builtin_amdgcn_readfirstlane(x);
+    if (x0 >= a.width) continue;  // past the last tile
+    const bool inside = x < a.width && tp.y < a.height;
+    const RawLookup<MIP> r = raw_lookup<MIP>(a, inside ? tp.pixel + 16 * (d - at) : tp.pixel);
+    if (__ballot(inside && differs(r)) == 0) found |= 1u << d;
+  }
+  const bool first = (found & ((1u << at) - 1u)) == 0u;
+  const int lane = lane_id();
+  uint32_t k0 = 0xffffffffu;
+  float w0 = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    // From the first lane: a lane outside the image has no taps of its own.
+    const uint32_t kk = (uint32_t)__builtin_amdgcn_readfirstlane((int)key[k]);
+    const float wk = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(weight[k])));
+    k0 = lane == k && first ? kk : k0;
+    w0 = lane == k && first ? wk : w0;
+    key[k] = 0xffffffffu;
+    weight[k] = 0.0f;
+  }
+  key[0] = k0;
+  weight[0] = w0;
+  return first ? found >> at : 0u;
+}
+
+// Channels [c0, c0 + N) of the upstream gradient summed over the strips of `strips`, in every
+// lane.
+template <int N>
+__device__ __forceinline__ void strip_sum(const DrTextureArgs& a, const TilePixel& tp,
+                                          uint32_t strips, const float* grad_out, int C, int c0,
+                                          float (&sum)[N]) {
+#pragma unroll
+  for (int c = 0; c < N; ++c) sum[c] = 0.0f;
+#pragma unroll 1
+  for (int d = 0; d < kStripTiles; ++d) {
+    if (((strips >> d) & 1u) == 0u) continue;  // uniform over the wave
+    if (tp.x + 16 * d < a.width && tp.y < a.height) {
+      float g[N];
+      load_channels<N>(grad_out + (tp.pixel + 16 * d) * C, C, c0, g);
+#pragma unroll
+      for (int c = 0; c < N; ++c) sum[c] += g[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < N; ++c) sum[c] = wave_masked_sum(sum[c], ~0ull);
+}
+
 // Channels per pass of the backward kernel for CHANNELS channels: 1-4 of them, or 0 for more, in
 // fours.
 template <int CHANNELS>
 constexpr int kPassChannels = CHANNELS == 0 ? 4 : CHANNELS;
 
+// The 2D kernels are held to 72 VGPRs: seven waves per SIMD (eight spill: texture forward and
+// backward at 8 x 1024^2 with a 1024^2 texture of 4 channels 493 -> 510 us; the cube-map kernels
+// spill at either, 239 -> 320 us at seven waves, and keep their own).
 template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : (CHANNELS > 0 ? 8 : 7)))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : 7))) void
 tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float* grad_uv,
                float* grad_uv_da, float* grad_bias) {
   constexpr int NC = kPassChannels<CHANNELS>;
@@ -395,6 +507,10 @@ tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float
   }
   if (grad_texels == nullptr) return;  // uniform over the workgroup
 
+  uint32_t strips = 0u;
+  constexpr bool kMip = FILTER == DR_FILTER_MIP_NEAREST || FILTER == DR_FILTER_MIP_LINEAR;
+  if constexpr (!CUBE) strips = shared_strips<kMip>(a, tp, tap_key, tap_weight);
+
   // Texel gradients, four channels per pass through the workgroup's table: tap k adds
   // g[c] * weight[k] to its texel row.
   float w_max = 0.0f;
@@ -404,7 +520,10 @@ tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float
   for (int c0 = 0; c0 < C; c0 += 4) {
     const int n = min(4, C - c0);
     float gc[4];
-    load_channels<4>(g, C, c0, gc);
+    if (strips != 0u)  // uniform over the wave
+      strip_sum<4>(a, tp, strips, grad_out, C, c0, gc);
+    else
+      load_channels<4>(g, C, c0, gc);
     // The largest |g[c] * weight[k]| of this lane (rounding is monotone, so the product of the
     // two largest factors is the largest product).
     float g_max = 0.0f;

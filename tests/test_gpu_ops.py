@@ -322,6 +322,42 @@ def test_texture_many_channels(channels, boundary, tex_batch):
         assert_grads_close(grads[:1], e_grads[:1])
 
 
+@pytest.mark.parametrize("channels", [1, 3, 4, 6])
+@pytest.mark.parametrize("filter_mode", FILTERS)
+@pytest.mark.parametrize("tex_batch", [1, 2])
+def test_texture_gradient_of_shared_lookups(channels, filter_mode, tex_batch):
+    # Strips of 16 x 4 pixels that share one lookup (background) add up over neighbouring tiles:
+    # constant images but for scattered pixels, strips that differ from their neighbours by one
+    # bit or by the sign of zero, NaN ones, partial tiles on both edges, two views apart.
+    gen = torch.Generator().manual_seed(channels)
+    h, w = 39, 150
+    tex = torch.randn(tex_batch, 9, 12, channels, generator=gen)
+    uv = torch.zeros(2, h, w, 2)
+    uv_da = torch.zeros(2, h, w, 4)
+    bias = torch.zeros(2, h, w) if "mipmap" in filter_mode and channels == 3 else None
+    uv[1] = 0.3
+    uv[0, :, 64:80, 0] = -0.0                      # a tile's strips of negative zeros
+    uv[0, 16:20, 96:112] = np.float32(1e-45).item()  # the smallest step from the background
+    uv[0, 20:24, 32:48, 0] = float("nan")
+    uv[1, 4:8, 16:32] = 0.7
+    uv_da[1, 8:12, 48:64] = 0.25
+    if bias is not None:
+        bias[1, 24:28, 80:96] = 1.5
+    some = torch.rand(2, h, w, generator=gen) < 0.01
+    uv[some] = torch.rand(int(some.sum()), 2, generator=gen)
+    weights = torch.randn(2, h, w, channels, generator=gen)
+    mip = "mipmap" in filter_mode
+    for boundary in BOUNDARIES:
+        def run(fn):
+            return lambda t: fn(t, uv.to(t.device), uv_da.to(t.device) if mip else None,
+                                filter_mode, boundary, None,
+                                mip_level_bias=None if bias is None else bias.to(t.device))
+
+        _, grads = grads_of(run(hip.texture), [tex], [weights], "cuda")
+        _, e_grads = grads_of(run(R.texture), [tex], [weights], "cpu")
+        assert_grads_close(grads, e_grads)
+
+
 @pytest.mark.parametrize("max_mip_level", [0, 2])
 def test_texture_max_mip_level(max_mip_level):
     tex, uv, uv_da = tex_scene()

@@ -201,7 +201,9 @@ def check(code: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call entry point ``name`` and raise ``RuntimeError`` on a nonzero status."""
-    check(getattr(load(), name)(*args), name)
+    code = getattr(_lib or load(), name)(*args)
+    if code != 0:
+        check(code, name)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -17,6 +17,7 @@ are kernels and cannot be differentiated again (``first_order``).
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 import weakref
 from collections.abc import Sequence
@@ -581,6 +582,17 @@ def interpolate(attr: Tensor, rast: Tensor, tri: Tensor, rast_db: Tensor | None,
 # ---------------------------------------------------------------------------------------------
 
 
+# The level sizes, offsets and C arrays of a chain depend on a few integers alone and are read,
+# never written: kept for the last shapes seen (some 15 us of a lookup's call otherwise).
+_PLANS_KEPT = 64
+
+
+@functools.lru_cache(maxsize=_PLANS_KEPT)
+def _chain_tables(height: int, width: int, max_mip_level: int | None, faces: int):
+    """(heights, widths, offsets) of the whole chain."""
+    return _tables(_chain_sizes(height, width, max_mip_level), faces)[:3]
+
+
 def _chain_sizes(height: int, width: int, max_mip_level: int | None) -> list[tuple[int, int]]:
     """Sizes of the box-filtered chain: halve rounding up until 1x1 (reference.py:433-446)."""
     sizes = [(height, width)]
@@ -600,6 +612,7 @@ def _tables(sizes, faces):
     return heights, widths, tuple(offsets), total
 
 
+@functools.lru_cache(maxsize=_PLANS_KEPT)
 def _level_arrays(heights, widths, offsets):
     n = len(heights)
     return ((ctypes.c_int32 * n)(*heights), (ctypes.c_int32 * n)(*widths),
@@ -648,9 +661,7 @@ class _MipChain(torch.autograd.Function):
 
 def _mip_chain(tex: Tensor, max_mip_level: int | None):
     faces = 6 if tex.ndim == 5 else 1
-    heights, widths, offsets, _ = _tables(_chain_sizes(tex.shape[-3], tex.shape[-2],
-                                                       max_mip_level), faces)
-    tables = (heights, widths, offsets)
+    tables = _chain_tables(tex.shape[-3], tex.shape[-2], max_mip_level, faces)
     return _MipChain.apply(tex, tables), tables
 
 
@@ -719,22 +730,27 @@ class _ChainTexture(torch.autograd.Function):
         return grad_tex, *grads[1:], None, None, None
 
 
-def _texture_args(texels, uv, uv_da, bias, tables, filter_mode, boundary_mode):
-    heights, widths, offsets = tables
+@functools.lru_cache(maxsize=_PLANS_KEPT)
+def _level_template(heights, widths, offsets) -> bytes:
+    """The bytes of a DrTextureArgs that holds the levels alone."""
     n = len(heights)
+    args = _lib.TextureArgs(num_levels=n)
+    args.level_height[:n] = heights
+    args.level_width[:n] = widths
+    args.level_offset[:n] = offsets
+    return bytes(args)
+
+
+def _texture_args(texels, uv, uv_da, bias, tables, filter_mode, boundary_mode):
+    n = len(tables[0])
     if n > _lib.MAX_LEVELS:
         raise ValueError(f"at most {_lib.MAX_LEVELS} mip levels are supported, got {n}.")
-    args = _lib.TextureArgs()
+    args = _lib.TextureArgs.from_buffer_copy(_level_template(*tables))
     args.texels = ptr(texels)
     args.tex_batch = texels.shape[0]
     args.channels = texels.shape[-1]
     args.num_texels = texels.shape[1]
-    args.num_levels = n
     args.faces = 6 if boundary_mode == "cube" else 1
-    for k in range(n):
-        args.level_height[k] = heights[k]
-        args.level_width[k] = widths[k]
-        args.level_offset[k] = offsets[k]
     args.uv = ptr(uv)
     args.uv_da = ptr(uv_da)
     args.bias = ptr(bias)
@@ -796,10 +812,9 @@ def texture(tex: Tensor, uv: Tensor, uv_da: Tensor | None, filter_mode: str, bou
         tables = (heights, widths, offsets)
     else:
         faces = 6 if tex.ndim == 5 else 1
-        heights, widths, offsets, _ = _tables(_chain_sizes(tex.shape[-3], tex.shape[-2],
-                                                           max_mip_level), faces)
-        return _ChainTexture.apply(tex, uv, uv_da, mip_level_bias, (heights, widths, offsets),
-                                   filter_mode, boundary_mode)
+        tables = _chain_tables(tex.shape[-3], tex.shape[-2], max_mip_level, faces)
+        return _ChainTexture.apply(tex, uv, uv_da, mip_level_bias, tables, filter_mode,
+                                   boundary_mode)
     return _Texture.apply(texels, uv, uv_da, mip_level_bias, tables, filter_mode, boundary_mode)
 
 

@@ -226,11 +226,11 @@ __global__ __launch_bounds__(256) void interp_fwd_wide_kernel(DrInterpolateArgs 
     for (int i = threadIdx.x; i < 256 * D; i += 256) {
       const int j = i / D, k = i - j * D;
       const int64_t at = place(j);
-      if (at < 0) continue;
+      const int c = a.diff[k];
+      if (at < 0 || c < 0 || c >= C) continue;
       const WidePixel p = s_pixel[j];
       float2 d = make_float2(0.0f, 0.0f);
       if (p.row[0] != kNoRow) {
-        const int c = a.diff[k];
         const float a0 = a.attr[(int64_t)p.row[0] * C + c], a1 = a.attr[(int64_t)p.row[1] * C + c];
         const float a2 = a.attr[(int64_t)p.row[2] * C + c];
         const float4 db = s_db[j];

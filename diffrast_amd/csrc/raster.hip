@@ -84,7 +84,8 @@ struct Workspace {
   uint4* record_bins;        // per record slot, what the bin pass reads (16 bytes, not the
                              // record's 64): tx0 | tx1 << 16, ty0 | ty1 << 16, the list of tile
                              // (0, 0) of its image and slab, and the bits of its triangle's
-                             // depth_lower_bound, which the bin pass copies into the entries
+                             // depth_lower_bound, which the bin pass copies into the entries;
+                             // a large triangle's ranges have their ends swapped
   // Tile lists: list tile * slabs + slab holds the binned triangles of that tile whose
   // nearest depth falls in depth slab `slab` of their image, so a tile's entries are one range
   // that runs near to far.

@@ -93,7 +93,7 @@ int dr_raster_order(const DrRasterGeometry* g, void* order, size_t order_bytes, 
 
 /* Visibility, first part: clears keys, orders the triangles of a large mesh spatially,
  * rasterizes triangles with a small bounding box directly, bins the others into 16x16 tiles
- * (counts and scan) and orders the tiles for the tile pass. Waits for the stream and returns
+ * (counts, and each list's place among the entries). Waits for the stream and returns
  * in counts[0..3] the number of setup workgroups (each with up to 256 binned triangles), tile
  * entries, workgroups of the tile pass (8 x the busy tiles of the XCD share with the most), and
  * tiles with at least one entry.
@@ -115,8 +115,8 @@ int dr_raster_visibility_start(const DrRasterGeometry* g, const uint64_t* prev_k
                                uint64_t* keys, void* workspace, size_t workspace_bytes,
                                uint32_t* host_counts, void* stream);
 
-/* Visibility, second part: fills the per-tile lists. entries holds counts[1] entries of 8
- * bytes (8-byte aligned): the lists of all tiles, tile by tile, near to far; an entry is a
+/* Visibility, second part: fills the per-tile lists and orders the tiles for the tile pass. entries holds counts[1] entries of 8
+ * bytes (8-byte aligned): the lists of all tiles, each tile's near to far; an entry is a
  * binned triangle's record number (uint32) and a lower bound of its depth (float32), by which
  * the tile pass skips triangles behind every key of a tile without reading their records. Nothing to do when counts[1] == 0. counts[1]
  * may also be a capacity larger than the lists: the kernel returns at once if they exceed it.

@@ -363,7 +363,7 @@ __device__ __forceinline__ uint32_t shared_strips(const DrTextureArgs& a, const 
     const int x0 = __builtin_amdgcn_readfirstlane(x);
     if (x0 >= a.width) continue;  // past the last tile
     const bool inside = x < a.width && tp.y < a.height;
-    const RawLookup<MIP> r = raw_lookup<MIP>(a, inside ? tp.pixel + 16 * (d - at) : tp.pixel);
+    const RawLookup<MIP> r = raw_lookup<MIP>(a, inside ? tp.pixel + 16 * (d - at) : 0);
     if (__ballot(inside && differs(r)) == 0) found |= 1u << d;
   }
   const bool first = (found & ((1u << at) - 1u)) == 0u;

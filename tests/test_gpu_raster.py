@@ -106,6 +106,7 @@ def test_mixed_triangle_sizes():
     (9, (97, 131), 1),     # one list workgroup, partial tiles
     (300, (64, 64), 1),    # depth slabs
     (40, (1100, 252), 2),  # lists of several workgroups, tile rows split between them
+    (70, (80, 560), 1),    # 175 tiles in a row-major run: triangles walked by lanes and by waves
     (2000, (160, 176), 140),  # dense: only triangles over more than 64 tiles are large
 ])
 def test_triangles_over_many_tiles(count, resolution, batch):
@@ -181,6 +182,9 @@ def rasterize_time(scene):
     # Twice the triangles, past a place per tile list: 4.21 / 0.50 ms before each had a place,
     # 0.80 / 0.50 with one.
     ((8000, 300, 1024), (4000, 300, 1024), 2.5),
+    # The same number close together, in the tiles of few workgroups: 0.75 / 0.33 ms while a
+    # wave walked one triangle at a time, 0.30 / 0.31 with each lane on its own.
+    ((12000, 64, 2048, 1 / 8), (12000, 64, 2048), 1.4),
 ])
 def test_large_triangles_take_time_by_their_number(scene, other, factor):
     assert rasterize_time(scattered(*scene)) < factor * rasterize_time(scattered(*other))

@@ -16,7 +16,7 @@
 //    small_pixels() pixel centres are rasterized right away (64-bit atomic min per covered
 //    pixel); the others are binned into 16x16 tiles. Per-tile counts gather in an LDS table of
 //    the workgroup before one global atomic per distinct tile.
-//    Triangles over more than kLargeTiles tiles only join a list of large triangles.
+//    Triangles over more than large_limit tiles only join a list of large triangles.
 // 3. One pass turns the tile counts (and the large triangles over each tile) into places for
 //    the tile lists; the bin pass reserves each workgroup's share of a tile's list with one
 //    global atomic and fills it. Each tile has one list per depth slab (the triangle's nearest
@@ -69,13 +69,20 @@ constexpr int kXcdShares = 8;        // XCDs of an MI355X: workgroup b runs on X
 constexpr int kCounters = 5;
 // A triangle over more tiles than this is binned by the workgroups that own the tiles, not by
 // its own thread, which walks its tiles one after another (two table steps per tile).
-// Dense meshes, whose many workgroups hide that walk, keep it up to kLargeTilesDense tiles:
-// every list workgroup reads every large triangle. Rasterize calls, this limit 8 against 64:
-// 224 triangles at 2160 x 3840 329 / 372 us, 512 at 1448^2 103 / 1452 us, 4096 at 2 x 2048^2
-// 350 / 1164 us; 1.31 M noisy ones at 8 x 1024^2: list and bin passes 348 / 184 us.
+// Every list workgroup reads every large triangle, so calls of many triangles, whose many
+// workgroups hide that walk, and those of many per tile keep it up to kLargeTilesMany tiles.
+// Rasterize calls, the limit 8 against 64, us, triangles of 48 pixels unless stated:
+//   224 over the whole of 2160 x 3840   184 / 216     3968 at 2 x 2048^2 (sphere)    286 / 1020
+//   4000 at 2048^2 (0.2 per tile)       203 / 350     16 k (1 per tile)              309 / 381
+//   24 k (1.5)                          372 / 386     32 k (2)                       430 / 382
+//   200 k (12)                         1356 / 600     24 k of 100 pixels (1.5)       528 / 907
+//   8000 at 1024^2 (2)                  227 / 275     24 k (6)                       310 / 166
+//   4000 at 8 x 1024^2 (1)              505 / 541     8000 (2; 64 k instances)       680 / 610
+//   4000 at 8 x 2048^2 (0.2)           1368 / 1440    16 k (1; 128 k instances)     2082 / 1829
 constexpr uint32_t kLargeTiles = 8;
-constexpr uint32_t kLargeTilesDense = 64;
-constexpr int64_t kLargeDenseFrom = (int64_t)1 << 18;  // triangle instances
+constexpr uint32_t kLargeTilesMany = 64;
+constexpr int64_t kLargePerTile = 2;                   // triangles per tile of an image
+constexpr int64_t kLargeInstances = (int64_t)1 << 15;  // triangles of all images
 
 struct Workspace {
   float4* records;           // binned triangles, kRecord float4 each: the three clip-space
@@ -136,8 +143,10 @@ int small_pixels(const DrRasterGeometry& g) {
   return g.ranges != nullptr ? kSmallPixelsRanges : kSmallPixelsDense;
 }
 
-uint32_t large_tiles_limit(const DrRasterGeometry& g) {
-  return g.num_instances < kLargeDenseFrom ? kLargeTiles : kLargeTilesDense;
+uint32_t large_tiles_limit(const DrRasterGeometry& g, int64_t image_tiles) {
+  return g.num_tri <= kLargePerTile * image_tiles && g.num_instances <= kLargeInstances
+             ? kLargeTiles
+             : kLargeTilesMany;
 }
 
 // Places in the list of large triangles: one each for the triangles of a smaller mesh; a larger
@@ -170,7 +179,7 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
   w.slabs = g.ranges != nullptr || g.num_tri <= kSlabsFrom * w.tiles_x * w.tiles_y ? 1
                                                                                   : kDepthSlabs;
   w.lists = w.tiles * w.slabs;
-  w.large_limit = large_tiles_limit(g);
+  w.large_limit = large_tiles_limit(g, (int64_t)w.tiles_x * w.tiles_y);
   w.large_places = large_list_places(g, w.lists);
   w.share_run = tile_run(g.batch, (uint32_t)std::min<int64_t>(w.tiles, 0xffffffffLL));
   const int64_t list_block = (int64_t)kListThreads * (w.slabs == 1 ? 1 : 4);

@@ -104,10 +104,12 @@ def test_mixed_triangle_sizes():
 
 @pytest.mark.parametrize("count,resolution,batch", [
     (9, (97, 131), 1),     # one list workgroup, partial tiles
-    (300, (64, 64), 1),    # depth slabs
+    (300, (64, 64), 1),    # many triangles per tile: large from 65 tiles, here none
+    (800, (144, 150), 1),  # the same in 90 tiles, with depth slabs
     (40, (1100, 252), 2),  # lists of several workgroups, tile rows split between them
     (70, (80, 560), 1),    # 175 tiles in a row-major run: triangles walked by lanes and by waves
-    (2000, (160, 176), 140),  # dense: only triangles over more than 64 tiles are large
+    (200, (160, 176), 170),   # many instances: large from 65 tiles, in the two views from 9
+    (2000, (160, 176), 140),  # many triangles per tile: large from 65 tiles in either
 ])
 def test_triangles_over_many_tiles(count, resolution, batch):
     gen = torch.Generator().manual_seed(31)
@@ -117,13 +119,14 @@ def test_triangles_over_many_tiles(count, resolution, batch):
         return
     pos = pos[torch.arange(batch) % 2].contiguous()
     ours = gpu_layers(pos, tri, resolution, 2)
-    each = gpu_layers(pos[:2], tri, resolution, 2)  # few instances: large from 9 tiles
+    each = gpu_layers(pos[:2], tri, resolution, 2)
     for (rast, db), (rast2, db2) in zip(ours, each):
         assert torch.equal(rast, rast2[torch.arange(batch) % 2])
         assert torch.equal(db, db2[torch.arange(batch) % 2])
     assert_layers_match(pos[:1], tri, resolution)
     # The same triangles as items of a range call (one list per tile).
-    ranges = torch.tensor([[0, 9], [9, 200], [500, 1500]], dtype=torch.int32)
+    ranges = torch.tensor([[0, 9], [9, count // 10], [count // 4, 3 * count // 4]],
+                          dtype=torch.int32)
     flat = pos[0].cuda()
     rast, _, _ = hip.rasterize_ranges(flat, tri.cuda(), resolution, True, ranges)
     ref, _ = R.rasterize_ranges(pos[0], tri, resolution, ranges)
@@ -185,6 +188,9 @@ def rasterize_time(scene):
     # The same number close together, in the tiles of few workgroups: 0.75 / 0.33 ms while a
     # wave walked one triangle at a time, 0.30 / 0.31 with each lane on its own.
     ((12000, 64, 2048, 1 / 8), (12000, 64, 2048), 1.4),
+    # No more time than for a third more: 1.83 / 0.68 ms while meshes of up to 2^18 instances
+    # had triangles over 9 tiles walked by every workgroup, 0.60 / 0.67 now.
+    ((200_000, 48, 2048), (270_000, 48, 2048), 1.4),
 ])
 def test_large_triangles_take_time_by_their_number(scene, other, factor):
     assert rasterize_time(scattered(*scene)) < factor * rasterize_time(scattered(*other))

@@ -199,6 +199,24 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
   return (uint64_t)hi << 32 | lo;
 }
 
+// Sum over the wave in float64, in every lane.
+__device__ __forceinline__ double wave_sum_f64(double v) {
+  auto moved = [](double x, auto move) {
+    const uint64_t bits = (uint64_t)__double_as_longlong(x);
+    return __longlong_as_double(
+        (long long)((uint64_t)move((uint32_t)(bits >> 32)) << 32 | move((uint32_t)bits)));
+  };
+  v += moved(v, [](uint32_t x) { return row_shr<1>(x); });
+  v += moved(v, [](uint32_t x) { return row_shr<2>(x); });
+  v += moved(v, [](uint32_t x) { return row_shr<4>(x); });
+  v += moved(v, [](uint32_t x) { return row_shr<8>(x); });
+  v += moved(v, [](uint32_t x) { return bcast15(x); });
+  v += moved(v, [](uint32_t x) { return bcast31(x); });
+  return moved(v, [](uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, DR_WAVE - 1);
+  });
+}
+
 template <int S, int N>
 __device__ __forceinline__ void run_step(float (&v)[N], bool take) {
 #pragma unroll

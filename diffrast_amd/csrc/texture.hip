@@ -326,6 +326,9 @@ __device__ __forceinline__ RawLookup<MIP> raw_lookup(const DrTextureArgs& a, int
 // 79 % background, 3 channels 164 -> 131 us; two 720 x 1280 with 16 channels 564 -> 474; eight
 // 1024^2, 38 % background, 4 channels 495 -> 493, 79 % of one texel lookup each 477 -> 292. Eight
 // tiles are 1-8 % slower (a wave of the background looks at all of them), two up to 12 %.
+// What it costs where no strip shares a lookup: the trilinear kernels of one to three channels
+// hold 63-72 VGPRs, seven waves, instead of 58-64 and eight (four 1024^2 images, backward alone:
+// 3 channels 564 -> 589 us, 1 channel 317 -> 330, texels a quarter of a pixel apart 296 -> 327).
 // Bit d of the result: the strip of the d-th tile to the right; 0: an ordinary wave.
 constexpr int kStripTiles = 4;
 
@@ -385,14 +388,16 @@ __device__ __forceinline__ uint32_t shared_strips(const DrTextureArgs& a, const 
   return first ? found >> at : 0u;
 }
 
-// Channels [c0, c0 + N) of the upstream gradient summed over the strips of `strips`, in every
-// lane.
+// `weight` times channels [c0, c0 + N) of the upstream gradient summed over the strips of
+// `strips`. Up to 256 values meet here that the row table would otherwise add in 64 bits, so the
+// sum is in float64: it is rounded once, after the tap's weight has scaled it.
 template <int N>
 __device__ __forceinline__ void strip_sum(const DrTextureArgs& a, const TilePixel& tp,
                                           uint32_t strips, const float* grad_out, int C, int c0,
-                                          float (&sum)[N]) {
+                                          float weight, float (&scaled)[N]) {
+  double sum[N];
 #pragma unroll
-  for (int c = 0; c < N; ++c) sum[c] = 0.0f;
+  for (int c = 0; c < N; ++c) sum[c] = 0.0;
 #pragma unroll 1
   for (int d = 0; d < kStripTiles; ++d) {
     if (((strips >> d) & 1u) == 0u) continue;  // uniform over the wave
@@ -400,11 +405,11 @@ __device__ __forceinline__ void strip_sum(const DrTextureArgs& a, const TilePixe
       float g[N];
       load_channels<N>(grad_out + (tp.pixel + 16 * d) * C, C, c0, g);
 #pragma unroll
-      for (int c = 0; c < N; ++c) sum[c] += g[c];
+      for (int c = 0; c < N; ++c) sum[c] += (double)g[c];
     }
   }
 #pragma unroll
-  for (int c = 0; c < N; ++c) sum[c] = wave_masked_sum(sum[c], ~0ull);
+  for (int c = 0; c < N; ++c) scaled[c] = (float)(wave_sum_f64(sum[c]) * (double)weight);
 }
 
 // Channels per pass of the backward kernel for CHANNELS channels: 1-4 of them, or 0 for more, in
@@ -412,11 +417,21 @@ __device__ __forceinline__ void strip_sum(const DrTextureArgs& a, const TilePixe
 template <int CHANNELS>
 constexpr int kPassChannels = CHANNELS == 0 ? 4 : CHANNELS;
 
-// The 2D kernels are held to 72 VGPRs: seven waves per SIMD (eight spill: texture forward and
-// backward at 8 x 1024^2 with a 1024^2 texture of 4 channels 493 -> 510 us; the cube-map kernels
-// spill at either, 239 -> 320 us at seven waves, and keep their own).
+// Waves per SIMD that the 2D kernels are held to. Trilinear lookups and more than four channels:
+// seven, 72 VGPRs, as many as the table's LDS allows (trilinear ones of 2-4 and of more than four
+// channels then spill two or three registers under wrapping; at eight, 64 VGPRs, texture forward
+// and backward at 8 x 1024^2 with a 1024^2 texture of 4 channels went from 493 to 510 us). The
+// others: eight, as nearly all take by themselves (4 channels, clamped, nearest level, two
+// 720 x 1280 images: 55 us at 66 VGPRs, 53 at 56). The cube-map kernels spill at either (239 -> 320 us
+// at seven) and keep their own.
+template <int CHANNELS, int FILTER>
+constexpr int bwd_waves() {
+  return CHANNELS == 0 || FILTER == DR_FILTER_MIP_LINEAR ? 7 : 8;
+}
+
 template <int CHANNELS, bool CUBE, int FILTER, int BOUNDARY>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CUBE ? 1 : 7))) void
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(CUBE ? 1 : bwd_waves<CHANNELS, FILTER>()))) void
 tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float* grad_uv,
                float* grad_uv_da, float* grad_bias) {
   constexpr int NC = kPassChannels<CHANNELS>;
@@ -513,6 +528,8 @@ tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float
 
   // Texel gradients, four channels per pass through the workgroup's table: tap k adds
   // g[c] * weight[k] to its texel row.
+  const float strip_weight = tap_weight[0];
+  if (strips != 0u) tap_weight[0] = 1.0f;  // strip_sum applies it
   float w_max = 0.0f;
 #pragma unroll
   for (int k = 0; k < 8; ++k)
@@ -521,7 +538,7 @@ tex_bwd_kernel(DrTextureArgs a, const float* grad_out, float* grad_texels, float
     const int n = min(4, C - c0);
     float gc[4];
     if (strips != 0u)  // uniform over the wave
-      strip_sum<4>(a, tp, strips, grad_out, C, c0, gc);
+      strip_sum<4>(a, tp, strips, grad_out, C, c0, strip_weight, gc);
     else
       load_channels<4>(g, C, c0, gc);
     // The largest |g[c] * weight[k]| of this lane (rounding is monotone, so the product of the

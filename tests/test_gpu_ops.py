@@ -358,6 +358,45 @@ def test_texture_gradient_of_shared_lookups(channels, filter_mode, tex_batch):
         assert_grads_close(grads, e_grads)
 
 
+def test_texture_gradient_of_shared_lookups_keeps_small_and_large_sums():
+    # Pixels that share one lookup (background) are summed before their tap weights apply.
+    # Gradients near the largest float whose weighted sum is far from it: the one texel that the
+    # lookup reaches has weight 1e-4.
+    h, w = 36, 150
+    tex = torch.zeros(1, 4, 4, 1)
+    uv = torch.full((1, h, w, 2), -0.49 / 4)
+    weights = torch.full((1, h, w, 1), 3e38)
+
+    def run(fn):
+        return lambda t: fn(t, uv.to(t.device), None, "linear", "zero", None)
+
+    _, grads = grads_of(run(hip.texture), [tex], [weights], "cuda")
+    assert bool(grads[0].isfinite().all())
+    x = -np.float32(0.49) / 4 * 4 - 0.5
+    expected = h * w * 3e38 * float(x - math.floor(x)) ** 2
+    assert abs(grads[0][0, 0, 0, 0].item() / expected - 1) < 1e-4
+
+    # Gradients that cancel: 2^20 and multiples of 1/8 (exact in float32), of one sign in the
+    # upper half of each strip of 16 x 4 pixels and the other in the lower half. A quarter of each
+    # reaches each of the four taps. The sum of a strip, or of four side by side, is rounded once
+    # (2^-24 of it) and so is each addition of one to the texel.
+    gen = torch.Generator().manual_seed(4)
+    uv = torch.zeros(1, h, w, 2)
+    sign = torch.where(torch.arange(h) % 4 < 2, 1.0, -1.0).view(1, h, 1, 1)
+    weights = sign * 2.0 ** 20 + torch.randint(-8, 9, (1, h, w, 1), generator=gen) / 8
+    tex = torch.zeros(1, 1, 1, 1)
+
+    def run_at_zero(fn):
+        return lambda t: fn(t, uv.to(t.device), None, "linear", "wrap", None)
+
+    _, grads = grads_of(run_at_zero(hip.texture), [tex], [weights], "cuda")
+    exact = weights.double()
+    groups = [exact[:, y:y + 4, x:x + 64].sum().abs().item()
+              for y in range(0, h, 4) for x in range(0, w, 64)]
+    bound = 2.0 ** -24 * sum(groups) * (4 * len(groups) + 2)
+    assert abs(grads[0].item() - exact.sum().item()) <= bound
+
+
 @pytest.mark.parametrize("max_mip_level", [0, 2])
 def test_texture_max_mip_level(max_mip_level):
     tex, uv, uv_da = tex_scene()

@@ -659,13 +659,14 @@ __device__ __forceinline__ float* level_of(float* texels, int64_t num_texels, in
          (L.off[lvl] + (int64_t)face * L.h[lvl] * L.w[lvl]) * C;
 }
 
-// Level k + 1 from level k, one thread per destination texel and channel, `blocks` workgroups
-// per (image, face).
+// Level k + 1 from level k, one thread per destination texel and channel of all images and faces:
+// `values` of them each, `count` (below 2^32, as any launch's threads) in all.
 __global__ __launch_bounds__(256) void mip_down(float* texels, int C, int64_t num_texels,
-                                                int faces, MipLevels L, int k, uint32_t blocks) {
-  const uint32_t which = blockIdx.x / blocks;
-  const uint32_t i = (blockIdx.x - which * blocks) * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)L.h[k + 1] * L.w[k + 1] * C) return;
+                                                int faces, MipLevels L, int k, uint32_t values,
+                                                uint32_t count) {
+  const uint32_t thread = blockIdx.x * blockDim.x + threadIdx.x;
+  if (thread >= count) return;
+  const uint32_t which = thread / values, i = thread - which * values;
   const int64_t image = which / (uint32_t)faces;
   const int face = (int)(which % (uint32_t)faces);
   down_value(level_of(texels, num_texels, C, L, k, image, face),
@@ -675,10 +676,11 @@ __global__ __launch_bounds__(256) void mip_down(float* texels, int C, int64_t nu
 
 // Adjoint of mip_down: one thread per source texel and channel.
 __global__ __launch_bounds__(256) void mip_up(float* grad, int C, int64_t num_texels, int faces,
-                                              MipLevels L, int k, uint32_t blocks) {
-  const uint32_t which = blockIdx.x / blocks;
-  const uint32_t i = (blockIdx.x - which * blocks) * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)L.h[k] * L.w[k] * C) return;
+                                              MipLevels L, int k, uint32_t values,
+                                              uint32_t count) {
+  const uint32_t thread = blockIdx.x * blockDim.x + threadIdx.x;
+  if (thread >= count) return;
+  const uint32_t which = thread / values, i = thread - which * values;
   const int64_t image = which / (uint32_t)faces;
   const int face = (int)(which % (uint32_t)faces);
   up_value(level_of(grad, num_texels, C, L, k, image, face),
@@ -699,7 +701,7 @@ __global__ __launch_bounds__(kMipTailThreads) void mip_down_tail(float* texels, 
     const float* src = level_of(texels, num_texels, C, L, lvl, image, face);
     float* dst = level_of(texels, num_texels, C, L, lvl + 1, image, face);
     const uint32_t count = (uint32_t)(L.h[lvl + 1] * L.w[lvl + 1] * C);
-    for (uint32_t i = threadIdx.x; i < count; i += kMipTailThreads)
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x)
       down_value(src, dst, C, L.h[lvl], L.w[lvl], L.w[lvl + 1], i);
     __syncthreads();  // the next level reads what the workgroup wrote
   }
@@ -715,7 +717,7 @@ __global__ __launch_bounds__(kMipTailThreads) void mip_up_tail(float* grad, int 
     float* src = level_of(grad, num_texels, C, L, lvl, image, face);
     const float* dst = level_of(grad, num_texels, C, L, lvl + 1, image, face);
     const uint32_t count = (uint32_t)(L.h[lvl] * L.w[lvl] * C);
-    for (uint32_t i = threadIdx.x; i < count; i += kMipTailThreads)
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x)
       up_value(src, dst, C, L.h[lvl], L.w[lvl], L.h[lvl + 1], L.w[lvl + 1], i);
     __syncthreads();  // the next level reads what the workgroup wrote
   }
@@ -943,6 +945,22 @@ void stage_elements(int C, const void* texels, const void* base, F f) {
 // 2048 to 16384 within 3 % of a step of 1500 x 1500 x 16: 722, 720 and 740 us).
 constexpr int64_t kMipTailValues = 4096;
 
+// Whether level k's values (per image and face) end the chain in one workgroup's levels. Not
+// where there are many tiny ones: 100 k images of 3 x 3, built and folded back, 67 us level by
+// level, 210 in workgroups of one wave; of 7 x 7 x 3 756 and 551, 16384 of 3 x 2 x 16 70 and 76.
+bool tail_level(int64_t values, int64_t images) {
+  return values <= kMipTailValues && (images <= 4096 || values > 128);
+}
+
+// Threads of a tail's workgroups: all of them while the workgroups are few enough to run at once
+// (two to a CU); more workgroups finish sooner with fewer threads each (4096 images of
+// 24 x 24 x 3: 341 us with 1024 threads, 225 with a thread per 16 values; 1024 images: 122 either).
+int tail_threads(const MipLevels& L, int k, int channels, int64_t images) {
+  if (images <= 512) return kMipTailThreads;
+  const int64_t values = (int64_t)L.h[k] * L.w[k] * channels;
+  return (int)(values / 16 / 64 + 1) * 64;  // at most 320
+}
+
 // Parts of a chain: part (k, G) builds levels k + 1 .. k + G, in one tile-stage launch when
 // G >= 2, else (G == 1) with mip_down; the part at index `tail`, if any, is the last, with
 // mip_down_tail.
@@ -952,7 +970,7 @@ struct MipPlan {
   int k[DR_MAX_LEVELS], G[DR_MAX_LEVELS];
 };
 
-MipPlan mip_plan(const MipLevels& L, int num_levels, int channels) {
+MipPlan mip_plan(const MipLevels& L, int num_levels, int channels, int64_t images) {
   MipPlan P{};
   P.tail = -1;
   for (int k = 0; k + 1 < num_levels;) {
@@ -961,7 +979,7 @@ MipPlan mip_plan(const MipLevels& L, int num_levels, int channels) {
            L.w[k] % (2 << G) == 0)
       ++G;
     if (G < 2) G = 1;
-    if (k + G + 1 < num_levels && (int64_t)L.h[k] * L.w[k] * channels <= kMipTailValues) {
+    if (k + G + 1 < num_levels && tail_level((int64_t)L.h[k] * L.w[k] * channels, images)) {
       P.tail = P.count;  // more than one launch otherwise
       G = num_levels - 1 - k;
     }
@@ -975,6 +993,24 @@ MipPlan mip_plan(const MipLevels& L, int num_levels, int channels) {
 
 int64_t stage_tiles(const MipLevels& L, int k, int G, int64_t images) {
   return images * (int64_t)(L.h[k] >> G) * (L.w[k] >> G);
+}
+
+// Whether every launch that builds the plan's levels (up: folds them back), and the copy of
+// level 0 where one is needed, has fewer than 2^32 threads: the runtime does not refuse every
+// larger one, but runs a part of its workgroups.
+bool launchable(const MipPlan& P, const MipLevels& L, int channels, int64_t images, bool up,
+                bool copied) {
+  constexpr int64_t kLimit = (int64_t)1 << 32;
+  auto values = [&](int k) { return images * L.h[k] * L.w[k] * channels + 255; };
+  if (copied && values(0) >= kLimit) return false;
+  for (int s = 0; s < P.count; ++s) {
+    const int k = P.k[s], G = P.G[s];
+    const int64_t threads = s == P.tail ? images * tail_threads(L, k, channels, images)
+                            : G >= 2    ? stage_tiles(L, k, G, images) * 256
+                                        : values(up ? k : k + 1);
+    if (threads >= kLimit) return false;
+  }
+  return true;
 }
 
 bool valid_levels(int num_levels, const int32_t* h, const int32_t* w, const int64_t* off) {
@@ -1115,12 +1151,14 @@ extern "C" int dr_mip_build(float* texels, const float* base, int32_t tex_batch,
       !valid_levels(num_levels, level_height, level_width, level_offset))
     return DR_ERR_ARGUMENT;
   const MipLevels L = copy_levels(num_levels, level_height, level_width, level_offset);
-  const MipPlan P = mip_plan(L, num_levels, channels);
   const int64_t images = (int64_t)tex_batch * faces;
+  const MipPlan P = mip_plan(L, num_levels, channels, images);
   const int64_t base_texels = (int64_t)faces * L.h[0] * L.w[0];
   if (base != nullptr && base_texels > num_texels) return DR_ERR_ARGUMENT;
   // Level 0 from `base`: the first tile stage copies it as it reads it; otherwise a copy first.
   const bool staged_copy = base != nullptr && P.count > 0 && P.G[0] >= 2 && P.tail != 0;
+  if (!launchable(P, L, channels, images, false, base != nullptr && !staged_copy))
+    return DR_ERR_ARGUMENT;
   if (base != nullptr && !staged_copy) {
     const int64_t count = (int64_t)tex_batch * base_texels * channels;
     mip_copy_base<<<blocks_for(count, 256), 256, 0, (hipStream_t)stream>>>(
@@ -1129,7 +1167,8 @@ extern "C" int dr_mip_build(float* texels, const float* base, int32_t tex_batch,
   for (int s = 0; s < P.count; ++s) {
     const int k = P.k[s], G = P.G[s];
     if (s == P.tail) {
-      mip_down_tail<<<(unsigned)images, kMipTailThreads, 0, (hipStream_t)stream>>>(
+      mip_down_tail<<<(unsigned)images, tail_threads(L, k, channels, images), 0,
+                      (hipStream_t)stream>>>(
           texels, channels, num_texels, faces, L, k, k + G);
       continue;
     }
@@ -1144,9 +1183,9 @@ extern "C" int dr_mip_build(float* texels, const float* base, int32_t tex_batch,
       });
       continue;
     }
-    const int64_t blocks = blocks_for((int64_t)L.h[k + 1] * L.w[k + 1] * channels, 256);
-    mip_down<<<(unsigned)(images * blocks), 256, 0, (hipStream_t)stream>>>(
-        texels, channels, num_texels, faces, L, k, (uint32_t)blocks);
+    const int64_t values = (int64_t)L.h[k + 1] * L.w[k + 1] * channels;
+    mip_down<<<blocks_for(images * values, 256), 256, 0, (hipStream_t)stream>>>(
+        texels, channels, num_texels, faces, L, k, (uint32_t)values, (uint32_t)(images * values));
   }
   return launch_status();
 }
@@ -1159,12 +1198,14 @@ extern "C" int dr_mip_build_backward(float* grad_texels, int32_t tex_batch, int3
       !valid_levels(num_levels, level_height, level_width, level_offset))
     return DR_ERR_ARGUMENT;
   const MipLevels L = copy_levels(num_levels, level_height, level_width, level_offset);
-  const MipPlan P = mip_plan(L, num_levels, channels);
   const int64_t images = (int64_t)tex_batch * faces;
+  const MipPlan P = mip_plan(L, num_levels, channels, images);
+  if (!launchable(P, L, channels, images, true, false)) return DR_ERR_ARGUMENT;
   for (int s = P.count - 1; s >= 0; --s) {
     const int k = P.k[s], G = P.G[s];
     if (s == P.tail) {
-      mip_up_tail<<<(unsigned)images, kMipTailThreads, 0, (hipStream_t)stream>>>(
+      mip_up_tail<<<(unsigned)images, tail_threads(L, k, channels, images), 0,
+                    (hipStream_t)stream>>>(
           grad_texels, channels, num_texels, faces, L, k, k + G);
       continue;
     }
@@ -1177,9 +1218,10 @@ extern "C" int dr_mip_build_backward(float* grad_texels, int32_t tex_batch, int3
       });
       continue;
     }
-    const int64_t blocks = blocks_for((int64_t)L.h[k] * L.w[k] * channels, 256);
-    mip_up<<<(unsigned)(images * blocks), 256, 0, (hipStream_t)stream>>>(
-        grad_texels, channels, num_texels, faces, L, k, (uint32_t)blocks);
+    const int64_t values = (int64_t)L.h[k] * L.w[k] * channels;
+    mip_up<<<blocks_for(images * values, 256), 256, 0, (hipStream_t)stream>>>(
+        grad_texels, channels, num_texels, faces, L, k, (uint32_t)values,
+        (uint32_t)(images * values));
   }
   return launch_status();
 }

@@ -76,5 +76,16 @@ def test_argument_checks_before_launch():
     widths = (ctypes.c_int32 * 2)(4, 2)
     offsets = (ctypes.c_int64 * 2)(0, 16)
     assert lib.dr_mip_build(1, None, 1, 3, 22, 1, 2, heights, widths, offsets, None) == 1001
+    # 2^32 threads or more in a launch: 2^24 workgroups of a tile stage, of one-wave workgroups
+    # for 2^26 images, of single values.
+    for size, images in ((4, 1 << 24), (13, 1 << 26), (3, 1 << 30)):
+        sizes = [size]
+        while sizes[-1] > 1:
+            sizes.append((sizes[-1] + 1) // 2)
+        n = len(sizes)
+        level, offset = (ctypes.c_int32 * n)(*sizes), (ctypes.c_int64 * n)()
+        assert lib.dr_mip_build(1, None, images, 1, 400, 1, n, level, level, offset, None) == 1001
+        assert lib.dr_mip_build_backward(1, images, 1, 400, 1, n, level, level, offset,
+                                         None) == 1001
     with pytest.raises(RuntimeError, match="invalid argument"):
         _lib.check(1001, "probe")

@@ -477,6 +477,8 @@ def test_mip_chain_tile_stages(shape):
     ((1, 96, 96, 5), 0), ((2, 32, 32, 17), 0),   # channels that do not come in fours
     ((3, 45, 30, 2), 0), ((1, 6, 24, 24, 3), 0),  # chains ending in one workgroup's levels
     ((1, 130, 70, 7), 0),                        # levels of their own before those
+    ((600, 7, 7, 3), 0), ((513, 17, 15, 16), 0),  # more images than workgroups run at once
+    ((4100, 3, 3, 1), 0), ((4097, 5, 9, 3), 0),  # more still: tiny levels on their own, or not
 ])
 def test_mip_chain_channels_and_tails(shape, offset):
     gen = torch.Generator().manual_seed(6)
@@ -495,6 +497,28 @@ def test_mip_chain_channels_and_tails(shape, offset):
         grads.append(whole.grad.cpu())
     # A base texel sums at most one product per level and axis weight: a few roundings.
     torch.testing.assert_close(grads[0], grads[1], atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("images,size", [(4_300_000, (3, 3)), (17_000_000, (2, 2))])
+def test_mip_chain_of_millions_of_tiny_images(images, size):
+    # A launch has fewer than 2^32 threads: fewer workgroups of 1024, or of 256, than there are
+    # images here (the runtime runs a part of a larger launch, without an error).
+    gen = torch.Generator().manual_seed(7)
+    few = torch.randn(100, *size, 1, generator=gen)
+    ref = [t.detach() for t in R.texture_construct_mip(few, None)]
+    leaf = few.requires_grad_()
+    weights = [torch.randn(l.shape, generator=gen) for l in ref]
+    sum((l * w).sum() for l, w in zip(R.texture_construct_mip(leaf, None), weights)).backward()
+
+    def many(t):
+        return t.detach().cuda().repeat(images // 100, 1, 1, 1)
+
+    tex = many(few).requires_grad_()
+    levels = hip.texture_construct_mip(tex, None)
+    for a, b in zip(levels, ref):
+        torch.testing.assert_close(a.detach(), many(b), atol=1e-6, rtol=1e-6)
+    grad, = torch.autograd.grad(levels, [tex], [many(w) for w in weights])
+    torch.testing.assert_close(grad, many(leaf.grad), atol=1e-5, rtol=1e-5)
 
 
 def test_texture_through_public_api_with_mip_stack():

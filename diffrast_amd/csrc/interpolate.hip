@@ -158,7 +158,7 @@ __device__ __forceinline__ float4 blend(float u, float v, float w, float4 a, flo
                      blend(u, v, w, a.z, b.z, c.z), blend(u, v, w, a.w, b.w, c.w));
 }
 
-// The forward pass for any channel count: a workgroup's 256 pixels (rows or 32 x 8 tiles) leave
+// The forward pass for more than four channels: a workgroup's 256 pixels (rows or 32 x 8 tiles) leave
 // their rows and barycentrics in LDS, then consecutive lanes take a pixel's channels in turn, V
 // (one, two or four of them) at a time, so that the attribute rows are read and the output is
 // written in whole lines. (One pixel per thread and four of its
@@ -512,6 +512,48 @@ uint32_t image_rows(const DrInterpolateArgs& a) {
              : (uint32_t)(a.attr_batch_stride / a.channels);
 }
 
+// The wide kernel over all images, in halves (of the images, then of an image's rows) where one
+// launch would have 2^32 threads or more.
+constexpr int64_t kMaxBlocks = ((int64_t)1 << 24) - 1;
+
+int forward_wide(const DrInterpolateArgs& a, float* out, float* out_da, uint32_t rows_per_image,
+                 bool tiles, hipStream_t st) {
+  constexpr int TW = kGatherTileWidth;
+  const int64_t pixels = (int64_t)a.batch * a.height * a.width;
+  const int64_t blocks = tiles ? pixel_slot_blocks<1, true, TW>(a.batch, a.height, a.width)
+                               : (pixels + 255) / 256;
+  if (blocks > kMaxBlocks && (a.batch > 1 || a.height > 1)) {
+    const bool images = a.batch > 1;
+    DrInterpolateArgs first = a, second = a;
+    if (images)
+      second.batch -= first.batch = a.batch / 2;
+    else
+      second.height -= first.height = a.height / 2;
+    const int64_t skipped = (int64_t)first.batch * first.height * a.width;
+    second.rast += 4 * skipped;
+    if (a.rast_db) second.rast_db += 4 * skipped;
+    if (images) second.attr += (int64_t)first.batch * a.attr_batch_stride;
+    const int status = forward_wide(first, out, out_da, rows_per_image, tiles, st);
+    if (status != DR_OK) return status;
+    return forward_wide(second, out + skipped * a.channels,
+                        out_da ? out_da + skipped * 2 * a.num_diff : nullptr, rows_per_image,
+                        tiles, st);
+  }
+  return with_element(a.channels, a.attr, out, [&](auto v) {
+    return with_derivatives(a.num_diff > 0, [&](auto diff) {
+      using V = decltype(v);
+      constexpr bool DIFF = decltype(diff)::value;
+      if (tiles)
+        interp_fwd_wide_kernel<V, true, DIFF>
+            <<<(unsigned)blocks, 256, 0, st>>>(a, out, out_da, rows_per_image);
+      else
+        interp_fwd_wide_kernel<V, false, DIFF>
+            <<<(unsigned)blocks, 256, 0, st>>>(a, out, out_da, rows_per_image);
+      return launch_status();
+    });
+  });
+}
+
 bool valid_args(const DrInterpolateArgs* a) {
   if (!a || a->batch < 0 || a->height <= 0 || a->width <= 0 || a->channels < 0) return false;
   if (a->num_tri < 0 || a->num_diff < 0 || a->num_vertices < 0) return false;
@@ -542,25 +584,8 @@ extern "C" int dr_interpolate_forward(const DrInterpolateArgs* a, float* out, fl
   // The index rows and attribute rows one image's pixels may gather.
   const int64_t rows = rows_per_image != 0 ? rows_per_image : args.num_vertices;
   const bool tiles = gather_tiles(12 * (int64_t)args.num_tri + 4 * rows * args.channels);
-  if (wide_channels(args.channels)) {
-    return with_element(args.channels, args.attr, out, [&](auto v) {
-      return with_derivatives(args.num_diff > 0, [&](auto diff) {
-        using V = decltype(v);
-        constexpr bool DIFF = decltype(diff)::value;
-        constexpr int TW = kGatherTileWidth;
-        const hipStream_t st = (hipStream_t)stream;
-        if (tiles)
-          interp_fwd_wide_kernel<V, true, DIFF>
-              <<<pixel_slot_blocks<1, true, TW>(args.batch, args.height, args.width), 256, 0,
-                 st>>>(args, out, da, rows_per_image);
-        else
-          interp_fwd_wide_kernel<V, false, DIFF>
-              <<<pixel_slot_blocks<1, false, TW>(args.batch, args.height, args.width), 256, 0,
-                 st>>>(args, out, da, rows_per_image);
-        return launch_status();
-      });
-    });
-  }
+  if (wide_channels(args.channels))
+    return forward_wide(args, out, da, rows_per_image, tiles, (hipStream_t)stream);
   return exact_channels(args.channels, [&](auto nc) {
     return with_derivatives(args.num_diff > 0, [&](auto diff) {
       constexpr int NC = decltype(nc)::value > 0 ? decltype(nc)::value : 1;  // 1-4 here

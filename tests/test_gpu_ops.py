@@ -96,6 +96,33 @@ def test_interpolate_many_channels(channels, offset, triangles):
         assert_grads_close(ours[2:], ref[2:])
 
 
+def test_interpolate_more_pixels_than_a_launch_has_threads():
+    # 16 images of 16400 x 16384, past 2^32 pixels: one thread each would be more than a launch
+    # holds. All background but for marked pixels, which must hold their blend in every part.
+    shape = (16, 16400, 16384)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 225e9:
+        pytest.skip("needs 206 GB of free GPU memory")
+    gen = torch.Generator().manual_seed(5)
+    attr = torch.randn(16, 3, 8, generator=gen)
+    marked = [(0, 0, 0), (7, 16399, 16383), (8, 0, 0), (15, 8200, 77), (15, 16399, 16382)]
+    try:
+        rast = torch.zeros(*shape, 4, device="cuda")
+        for at in marked:
+            rast[at] = torch.tensor([0.25, 0.5, 0.1, 1.0])
+        tri = torch.tensor([[0, 1, 2]], dtype=torch.int32, device="cuda")
+        out, _ = hip.interpolate(attr.cuda(), rast, tri, None, [])
+        del rast
+        for at in marked:
+            b = at[0]
+            expected = 0.25 * attr[b, 0] + 0.5 * attr[b, 1] + 0.25 * attr[b, 2]
+            torch.testing.assert_close(out[at].cpu(), expected, atol=1e-6, rtol=1e-6)
+        assert not out[:, ::1640, 100:200].any() and not out[15, 16399, 16383].any()
+    finally:
+        rast = out = None
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("layout", ["shared", "per_view"])
 @pytest.mark.parametrize("diff", [[], [0, 2, 3], [1, 1]])
 def test_interpolate_gradients(layout, diff):

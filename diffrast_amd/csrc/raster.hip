@@ -2017,8 +2017,8 @@ static int queue_visibility_start(const DrRasterGeometry* g, const uint64_t* pre
 constexpr int64_t kPlainTileGrid = 1 << 16;
 
 // Launches the tile pass so that it covers every busy tile whatever `requested` is. A grid of
-// at least one workgroup per tile of the largest share (`requested` 0 or at least 8 x that, and
-// then at most kPlainTileGrid tiles) runs the plain kernel, one tile per workgroup. Any smaller grid
+// at least one workgroup per tile (`requested` 0 or at least the tiles) runs, up to kPlainTileGrid
+// tiles, the plain kernel with a workgroup per tile of every share's length. Any smaller grid
 // runs the looping kernel: `requested` workgroups (0: one per tile), rounded up to a multiple
 // of 8 and kept below 2^24, each taking every (grid / 8)-th busy tile of its XCD share. So a
 // grid sized before the busy tiles were known, or sized wrongly by a caller, loses no tile.
@@ -2027,7 +2027,7 @@ static void launch_tile_pass(const DrRasterGeometry& g, const uint64_t* prev, ui
                              uint32_t requested, hipStream_t s) {
   const int64_t bound = tile_grid_bound(ws);
   const int64_t limit = ((int64_t)1 << 24) - kXcdShares;
-  const bool full = requested == 0 || (int64_t)requested >= bound;
+  const bool full = requested == 0 || (int64_t)requested >= ws.tiles;
   if (full && ws.tiles <= kPlainTileGrid) {
     raster_tile_kernel<false><<<(int)bound, 256, 0, s>>>(g, prev, keys, ws, entries, capacity);
     return;

@@ -115,11 +115,13 @@ int dr_raster_visibility_start(const DrRasterGeometry* g, const uint64_t* prev_k
                                uint64_t* keys, void* workspace, size_t workspace_bytes,
                                uint32_t* host_counts, void* stream);
 
-/* Visibility, second part: fills the per-tile lists and orders the tiles for the tile pass. entries holds counts[1] entries of 8
- * bytes (8-byte aligned): the lists of all tiles, each tile's near to far; an entry is a
- * binned triangle's record number (uint32) and a lower bound of its depth (float32), by which
- * the tile pass skips triangles behind every key of a tile without reading their records. Nothing to do when counts[1] == 0. counts[1]
- * may also be a capacity larger than the lists: the kernel returns at once if they exceed it.
+/* Visibility, second part: fills the per-tile lists and orders the tiles for the tile pass.
+ * entries holds counts[1] entries of 8 bytes (8-byte aligned): the lists of all tiles, each
+ * tile's near to far where it has lists by depth; an entry is a binned triangle's record number
+ * (uint32) and a lower bound of its depth (float32), by which the tile pass skips triangles
+ * behind every key of a tile without reading their records. To be called once per start that
+ * its entries fit. Nothing to do when counts[1] == 0. counts[1] may also be a capacity larger
+ * than the lists: the kernel returns at once if they exceed it.
  * (The reference's pure-PyTorch visibility tests every triangle at every pixel,
  * reference.py:368-397; its Triton path bins triangles into tile chunks,
  * _triton_rasterize.py:371-424, and keeps the nearest per pixel in _tile_kernel,
@@ -130,7 +132,7 @@ int dr_raster_visibility_bin(const DrRasterGeometry* g, void* workspace, size_t 
 /* Visibility, third part: rasterizes the binned triangles tile by tile into keys, after
  * dr_raster_visibility_bin with the same entries and counts. Nothing to do when
  * counts[1] == 0. counts[2] is the pass's grid: 0, or at least one workgroup per 16x16 tile,
- * runs one workgroup per tile when that is at most 65536 workgroups; any smaller grid (rounded
+ * runs one workgroup per tile for at most 65536 tiles; any smaller grid (rounded
  * up to a multiple of 8) runs a looping kernel in which each workgroup takes every
  * (grid / 8)-th busy tile of its XCD share. Either way every tile is covered, whatever
  * counts[2] and counts[3] hold; counts[2] as dr_raster_visibility_begin returns it is the

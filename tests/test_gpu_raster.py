@@ -819,7 +819,8 @@ def test_visibility_with_entry_buffer_queued_before_the_counts(resolution):
             assert torch.equal(keys, expected), (layer, capacity)
             # The one-call form: lists that do not fit go through the overflow pass; a tile
             # pass of fewer workgroups than busy tiles loops over them.
-            for groups in (0, 8, 24, counts[2]):
+            # (One workgroup per tile: no loop.)
+            for groups in (0, 8, 24, counts[2], 3 * -(-resolution[0] // 16) * -(-resolution[1] // 16)):
                 keys, got = _keys_one_call(pos, tri, resolution, capacity, groups, prev)
                 assert got == counts, (layer, capacity, groups)
                 assert torch.equal(keys, expected), (layer, capacity, groups)

@@ -53,7 +53,8 @@ __device__ __forceinline__ void atomic_add(float* p, float v) { unsafeAtomicAdd(
 // N consecutive floats at p, in one memory instruction for up to four of them. The copies state
 // no more than a float's alignment, which is all that this target's wide global loads and stores
 // need; a test of the address for a scalar path beside a wide one made the compiler split the
-// last access that the two have in common (texture forward at 8 x 1024^2, 4 channels: 127 -> 112 us).
+// last access that the two have in common (texture forward at 8 x 1024^2, 4 channels: 127 ->
+// 112 us).
 template <int N>
 __device__ __forceinline__ void load_floats(const float* p, float (&v)[N]) {
   __builtin_memcpy(v, p, sizeof(v));
@@ -276,10 +277,16 @@ __device__ __forceinline__ int64_t xcd_order(int64_t block, int64_t blocks) {
 // every eighth. With a batch of at least 8 each XCD takes one run, whole images that differ
 // little in work; with fewer images an eighth of them would be a band of an image, empty for
 // one XCD and the middle of the object for another, so each XCD takes kTileRuns bands.
-// One run against 16 of them (2 and 4 lie between or worse, 8 within 2 %): texture forward and
-// backward on one 1080 x 1920 image 205 -> 171 us, on two 720 x 1280 with 16 channels 1114 ->
-// 1001; rasterize forward and backward of 327 k triangles at 2048^2 335 -> 300; of 1.31 M at
-// 2 x 1024^2 362 -> 347; 224 triangles at 2160 x 3840 300 -> 303.
+// One run against 16 of them, kernels alone in us (2 to 8 lie between or are worse):
+//   tile pass                one 1080 x 1920 image 42 -> 18; 224 triangles at 2160 x 3840 109 -> 86
+//   texture backward         one 1080 x 1920 image 123 -> 108; 4 x 512^2 52 -> 57
+//   resolve backward         1 M triangles at 1080 x 1920 53 -> 27, 327 k at 2048^2 70 -> 59; 224
+//                            at 2160 x 3840 103 -> 122
+//   interpolate backward     one 1080 x 1920 image 58 -> 37; 16 channels at 1448^2 82 -> 55, at
+//                            4 x 512^2 52 -> 55, at 4 x 768^2 117 -> 127
+//   antialias (pairs, blend, backward)  4 x 1001 x 999 109 -> 105, 2 x 1024^2 118 -> 103; with
+//                            everything out of the caches 116 -> 110 and 135 -> 116
+// (One run is better where four images of a round object give each XCD a symmetric half.)
 constexpr int kXcds = 8;
 constexpr int kTileRuns = 16;
 __host__ __device__ __forceinline__ uint32_t tile_run(int batch, uint32_t tiles) {

@@ -84,7 +84,8 @@ constexpr int kGatherTileWidth = 32;
 // PPT pixels per thread, in rows or tiles (pixel_slots). The pixels' loads go out level by
 // level -- rast, then the triangles' index rows, then the attribute rows -- so that a thread
 // waits once per level for all its pixels, not once per pixel: the gathers are latency-bound.
-// NC: the channel count, 1-4 (interp_fwd_wide_kernel takes the others). DIFF: out_da is written (num_diff > 0); without it the kernel holds no derivative state.
+// NC: the channel count, 1-4 (interp_fwd_wide_kernel takes the others). DIFF: out_da is written
+// (num_diff > 0); without it the kernel holds no derivative state.
 template <int NC, int PPT, bool TILES, bool DIFF>
 __global__ __launch_bounds__(256) void interp_fwd_kernel(DrInterpolateArgs a,
                                                          float* __restrict__ out,
@@ -158,13 +159,13 @@ __device__ __forceinline__ float4 blend(float u, float v, float w, float4 a, flo
                      blend(u, v, w, a.z, b.z, c.z), blend(u, v, w, a.w, b.w, c.w));
 }
 
-// The forward pass for more than four channels: a workgroup's 256 pixels (rows or 32 x 8 tiles) leave
-// their rows and barycentrics in LDS, then consecutive lanes take a pixel's channels in turn, V
-// (one, two or four of them) at a time, so that the attribute rows are read and the output is
-// written in whole lines. (One pixel per thread and four of its
-// channels at a time, at 4 x 512^2 with 16 channels: 82 us, a store instruction touching 64
-// lines; this one 17 us, 5.0 TB/s. With 8 channels, 8 x 1024^2 and 1.31 M triangles, forward
-// and backward 306 -> 288 us; up to 4 channels a pixel per thread is as fast or faster.)
+// The forward pass for more than four channels: a workgroup's 256 pixels (rows or 32 x 8 tiles)
+// leave their rows and barycentrics in LDS, then consecutive lanes take a pixel's channels in
+// turn, V (one, two or four of them) at a time, so that the attribute rows are read and the output
+// is written in whole lines. (One pixel per thread and four of its channels at a time, at
+// 4 x 512^2 with 16 channels: 82 us, a store instruction touching 64 lines; this one 17 us,
+// 5.0 TB/s. With 8 channels, 8 x 1024^2 and 1.31 M triangles, forward and backward 306 -> 288 us;
+// up to 4 channels a pixel per thread is as fast or faster.)
 template <class V, bool TILES, bool DIFF>
 __global__ __launch_bounds__(256) void interp_fwd_wide_kernel(DrInterpolateArgs a,
                                                               float* __restrict__ out,
@@ -194,31 +195,29 @@ __global__ __launch_bounds__(256) void interp_fwd_wide_kernel(DrInterpolateArgs 
   };
   const int C = a.channels;
   const int per = C / (int)(sizeof(V) / 4);  // elements per pixel
-  if (per > 0) {
-    // Element i of the workgroup is element e of pixel j; a step of 256 elements moves them by
-    // (dj, de).
-    const int dj = 256 / per, de = 256 % per;
-    int j = (int)threadIdx.x / per, e = (int)threadIdx.x % per;
-    const V* attr = reinterpret_cast<const V*>(a.attr);
-    V* o = reinterpret_cast<V*>(out);
+  // Element i of the workgroup is element e of pixel j; a step of 256 elements moves them by
+  // (dj, de).
+  const int dj = 256 / per, de = 256 % per;
+  int j = (int)threadIdx.x / per, e = (int)threadIdx.x % per;
+  const V* attr = reinterpret_cast<const V*>(a.attr);
+  V* o = reinterpret_cast<V*>(out);
 #pragma unroll 2
-    for (int step = 0; step < per; ++step) {
-      const WidePixel p = s_pixel[j];
-      const int64_t at = place(j);
-      const bool covered = p.row[0] != kNoRow;
-      V r = {};
-      if (covered) {
-        const V a0 = attr[(int64_t)p.row[0] * per + e], a1 = attr[(int64_t)p.row[1] * per + e];
-        const V a2 = attr[(int64_t)p.row[2] * per + e];
-        r = blend(p.u, p.v, 1.0f - p.u - p.v, a0, a1, a2);
-      }
-      if (at >= 0) o[at * per + e] = r;
-      j += dj;
-      e += de;
-      if (e >= per) {
-        e -= per;
-        ++j;
-      }
+  for (int step = 0; step < per; ++step) {
+    const WidePixel p = s_pixel[j];
+    const int64_t at = place(j);
+    const bool covered = p.row[0] != kNoRow;
+    V r = {};
+    if (covered) {
+      const V a0 = attr[(int64_t)p.row[0] * per + e], a1 = attr[(int64_t)p.row[1] * per + e];
+      const V a2 = attr[(int64_t)p.row[2] * per + e];
+      r = blend(p.u, p.v, 1.0f - p.u - p.v, a0, a1, a2);
+    }
+    if (at >= 0) o[at * per + e] = r;
+    j += dj;
+    e += de;
+    if (e >= per) {
+      e -= per;
+      ++j;
     }
   }
   if constexpr (DIFF) {
@@ -588,7 +587,8 @@ extern "C" int dr_interpolate_forward(const DrInterpolateArgs* a, float* out, fl
     return forward_wide(args, out, da, rows_per_image, tiles, (hipStream_t)stream);
   return exact_channels(args.channels, [&](auto nc) {
     return with_derivatives(args.num_diff > 0, [&](auto diff) {
-      constexpr int NC = decltype(nc)::value > 0 ? decltype(nc)::value : 1;  // 1-4 here
+      // 1-4 channels come here; the case of more (0) has to compile.
+      constexpr int NC = decltype(nc)::value > 0 ? decltype(nc)::value : 1;
       constexpr bool DIFF = decltype(diff)::value;
       constexpr int PPT = 2;  // pixels per thread
       constexpr int TW = kGatherTileWidth;

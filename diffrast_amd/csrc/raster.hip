@@ -62,7 +62,7 @@ constexpr int kOrderMinTris = 8192;  // smaller meshes keep their own order
 constexpr int kTileSlots = 1024;     // LDS table of a workgroup's tiles
 constexpr int kRecord = 4;           // float4 per binned triangle record (one 64-byte line)
 constexpr int kDepthSlabs = 16;      // tile lists per tile, by the triangle's nearest depth
-                                     // (dense views; range mode keeps one list per tile)
+                                     // (range mode and sparse meshes keep one list per tile)
 constexpr int64_t kSlabsFrom = 8;    // triangles per tile from which instanced meshes use them
 constexpr int kRangeParts = 64;      // workgroups per image in the depth span reduction
 constexpr int kXcdShares = 8;        // XCDs of an MI355X: workgroup b runs on XCD b mod 8
@@ -130,7 +130,7 @@ struct Workspace {
   int depth_ranges;
   int list_blocks;
   int record_blocks;          // setup workgroups; each owns 256 record slots
-  int slabs;                  // tile lists per tile: kDepthSlabs, or 1 in range mode
+  int slabs;                  // tile lists per tile: kDepthSlabs, or 1 (layout)
   uint32_t share_run;         // consecutive tiles of one XCD share of the tile pass
   uint32_t large_limit;       // a triangle over more tiles than this is a large one
   uint32_t large_places;      // places in the list of them
@@ -173,9 +173,15 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
   // Range mode keeps one list per tile: its items' triangles mostly take the small-triangle path,
   // so the near-to-far slabs gain its tile pass nothing, while their lists (clears, scans) and
   // the depth span they need cost 0.2 ms per step of four layers of 256 items at 512 x 512.
-  // So do meshes of few triangles per tile, whose lists fit one chunk of the tile pass in most
-  // tiles: the slabs order chunks (20 k triangles at 8 x 1024^2, 5 per tile: rasterize 283 us
-  // with slabs, 259 without; at 20 per tile 474 and 495).
+  // So do meshes of few triangles per tile of an image: what the slabs gain is an order of the
+  // entries, which matters where many overlap, and sixteen lists per tile crowd the workgroups'
+  // tables of lists. Rasterize calls, slabs against one list, us:
+  //   spread over the image:  20 k at 8 x 1024^2 283 / 264, 5 k at 4 x 512^2 151 / 88, 2000 of 40
+  //     pixels at 256^2 243 / 101, 100 k of 40 pixels at 2048^2 427 / 347, 20 shells of 5 k at
+  //     2048^2 620 / 350; but at 20 triangles per tile 474 / 495
+  //   all in a hundredth of the image:  100 k of 12 pixels at 2048^2 121 / 159, 130 k of 10 pixels
+  //     122 / 149; the 20 shells at 0.3 of their size, 4 x 2048^2 280 / 300
+  // (The lists' lengths would tell these apart, but they are known only once the lists are made.)
   w.slabs = g.ranges != nullptr || g.num_tri <= kSlabsFrom * w.tiles_x * w.tiles_y ? 1
                                                                                   : kDepthSlabs;
   w.lists = w.tiles * w.slabs;
@@ -971,9 +977,9 @@ __global__ __launch_bounds__(256) void raster_setup_kernel(DrRasterGeometry g,
 //
 // The lists' places among the entries, and the tile pass's order: heavy tiles first within each
 // XCD's share. The tile pass takes the busy tiles in their XCD shares' order (its workgroups of
-// XCD k take share k), within a share the tiles with the most binned triangles first, so that the longest workgroups do not
-// start last: a counting sort by entry count in kWorkClasses classes of 32 entries. The order
-// within a class is free: tiles are independent.
+// XCD k take share k), within a share the tiles with the most binned triangles first, so that the
+// longest workgroups do not start last: a counting sort by entry count in kWorkClasses classes of
+// 32 entries. The order within a class is free: tiles are independent.
 
 // The XCD share of tile i: runs of tiles in turn (tile_run).
 __device__ __forceinline__ int xcd_share(const Workspace& ws, int64_t i) {
@@ -987,7 +993,7 @@ __device__ __forceinline__ int xcd_share(const Workspace& ws, int64_t i) {
 // side; the others by the whole wave one after another, 64 tiles of the shared rows at once.
 // Large triangles are few next to the tiles they cover, and a workgroup passes over all of them
 // in a fraction of the time one thread would walk one's tiles. Whole waves call this.
-// (Lanes' walks against the wave's alone, 64 pixels a triangle: 20 k in a 256th of 2048^2, whose
+// (Lanes' walks against the wave's alone, 64 pixels a triangle: 20 k in a 64th of 2048^2, whose
 // tiles belong to few workgroups, rasterize 984 -> 388 us; 4000 in a sixth of it 176 -> 171. As
 // many tiles as triangles, not half: 2000 of 400 pixels on 1024^2 438 -> 461, at half 442.)
 template <typename F>
@@ -1047,12 +1053,12 @@ __device__ __forceinline__ void large_tiles(const Workspace& ws, int64_t first_l
 }
 
 // One workgroup per PER lists a thread (whole tiles: one list each with PER = 1, else four
-// threads' lists): the large triangles over each list are counted in LDS, a scan over the workgroup's lists and one
-// addition to the entry count give every list its place -- a tile's lists in one range, near to
-// far; where the workgroup's ranges lie among the others' does not matter -- and each tile's
-// work class joins the class counts of its XCD share. The last workgroup to finish turns those
-// into the classes' first positions. (A three-phase scan of the lists, a pass for the classes
-// and one for the cursors before: five launches of 2-5 us each; one now.)
+// threads' lists): the large triangles over each list are counted in LDS, a scan over the
+// workgroup's lists and one addition to the entry count give every list its place -- a tile's
+// lists in one range, near to far; where the workgroup's ranges lie among the others' does not
+// matter -- and each tile's work class joins the class counts of its XCD share. The last workgroup
+// to finish turns those into the classes' first positions. (A three-phase scan of the lists, a
+// pass for the classes and one for the cursors before: five launches of 2-5 us each; one now.)
 template <int PER>
 __global__ __launch_bounds__(kListThreads) void raster_list_kernel(Workspace ws) {
   constexpr int kListBlock = PER * kListThreads;

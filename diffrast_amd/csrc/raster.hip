@@ -81,7 +81,7 @@ constexpr int kCounters = 5;
 //   4000 at 8 x 2048^2 (0.2)           1368 / 1440    16 k (1; 128 k instances)     2082 / 1829
 constexpr uint32_t kLargeTiles = 8;
 constexpr uint32_t kLargeTilesMany = 64;
-constexpr int64_t kLargePerTile = 2;                   // triangles per tile of an image
+constexpr int64_t kLargePerTile = 2;                   // triangles of all images per tile of theirs
 constexpr int64_t kLargeInstances = (int64_t)1 << 15;  // triangles of all images
 
 struct Workspace {
@@ -143,10 +143,9 @@ int small_pixels(const DrRasterGeometry& g) {
   return g.ranges != nullptr ? kSmallPixelsRanges : kSmallPixelsDense;
 }
 
-uint32_t large_tiles_limit(const DrRasterGeometry& g, int64_t image_tiles) {
-  return g.num_tri <= kLargePerTile * image_tiles && g.num_instances <= kLargeInstances
-             ? kLargeTiles
-             : kLargeTilesMany;
+uint32_t large_tiles_limit(const DrRasterGeometry& g, int64_t tiles) {
+  return g.num_instances <= std::min(kLargePerTile * tiles, kLargeInstances) ? kLargeTiles
+                                                                             : kLargeTilesMany;
 }
 
 // Places in the list of large triangles: one each for the triangles of a smaller mesh; a larger
@@ -185,7 +184,7 @@ Workspace layout(const DrRasterGeometry& g, char* base) {
   w.slabs = g.ranges != nullptr || g.num_tri <= kSlabsFrom * w.tiles_x * w.tiles_y ? 1
                                                                                   : kDepthSlabs;
   w.lists = w.tiles * w.slabs;
-  w.large_limit = large_tiles_limit(g, (int64_t)w.tiles_x * w.tiles_y);
+  w.large_limit = large_tiles_limit(g, w.tiles);
   w.large_places = large_list_places(g, w.lists);
   w.share_run = tile_run(g.batch, (uint32_t)std::min<int64_t>(w.tiles, 0xffffffffLL));
   const int64_t list_block = (int64_t)kListThreads * (w.slabs == 1 ? 1 : 4);

@@ -167,14 +167,17 @@ def scattered(count, pixels, side, region=1.0):
     return pos.cuda(), torch.arange(3 * count, dtype=torch.int32).view(-1, 3).cuda(), (side, side)
 
 
-def rasterize_time(scene):
+def rasterize_time(scene, ranges=None):
     """Time of one rasterize call of the scene (ms), of ten queued together."""
     times = []
     for _ in range(4):  # the first learns the sizes
         start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
         start.record()
         for _ in range(10):
-            hip.rasterize(*scene, False)
+            if ranges is None:
+                hip.rasterize(*scene, False)
+            else:
+                hip.rasterize_ranges(scene[0][0], *scene[1:], False, ranges)
         end.record()
         torch.cuda.synchronize()
         times.append(start.elapsed_time(end) / 10)
@@ -194,6 +197,14 @@ def rasterize_time(scene):
 ])
 def test_large_triangles_take_time_by_their_number(scene, other, factor):
     assert rasterize_time(scattered(*scene)) < factor * rasterize_time(scattered(*other))
+
+
+def test_large_triangles_of_a_range_take_no_longer_than_alone():
+    # What counts is how many triangles are drawn, not how many the mesh has.
+    pos, tri, size = scattered(4000, 48, 2048)
+    many = tri.repeat(50, 1)
+    alone = rasterize_time((pos, tri, size))
+    assert rasterize_time((pos, many, size), torch.tensor([[4000, 4000]])) < 1.3 * alone
 
 
 def test_large_mesh_in_spatial_order_keeps_index_tie_break():

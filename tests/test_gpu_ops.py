@@ -618,7 +618,7 @@ def test_edge_neighbours_of_a_closed_mesh():
     assert torch.equal(nbr.long(), R.edge_neighbours(tri))
 
 
-@pytest.mark.parametrize("channels", [1, 3, 4, 20])
+@pytest.mark.parametrize("channels", [1, 3, 4, 5, 6, 7, 8, 20])
 @pytest.mark.parametrize("mesh", [{}, {"w_range": (-1.0, 2.0)}, {"z_range": 2.0, "xy_range": 3.0}])
 def test_antialias_matches_oracle(channels, mesh):
     pos, tri, rast, color, weights = aa_scene(channels=channels, **mesh)

@@ -164,11 +164,13 @@ __device__ __forceinline__ void wide_value(const WideLevel<CUBE>& W, const float
   }
 }
 
-// More than four channels, N of them (4, 2 or 1: a divisor of the count) to a lane: each thread
-// works out one pixel's taps, then consecutive lanes take a pixel's channels in turn, so that
-// texels and output go in whole lines and the taps are worked out once. (A pixel per thread and
-// four channels at a time, two 720 x 1280 images with 16 channels: 180 us; this one 60.)
-template <int N, bool CUBE, int FILTER, int BOUNDARY>
+// More than four channels, four to a lane: each thread works out one pixel's taps, then consecutive
+// lanes take a pixel's channels in turn, so that texels and output go in whole lines and the taps
+// are worked out once. (A pixel per thread and four channels at a time, two 720 x 1280 images with
+// 16 channels: 180 us; this one 60.) A last group past the end moves back over the one before, and
+// the channels that both have are written twice, the same. (Lanes of one or two channels for counts
+// that four does not divide, trilinear, two 720 x 1280 images: 5 channels 48 us, 30 this way; 7 64 and 31; 10 52 and 39.)
+template <bool CUBE, int FILTER, int BOUNDARY>
 __global__ __launch_bounds__(256) void tex_fwd_wide_kernel(DrTextureArgs a,
                                                            float* __restrict__ out) {
   __shared__ WideLookup<CUBE> s_lookup[256];
@@ -204,14 +206,16 @@ __global__ __launch_bounds__(256) void tex_fwd_wide_kernel(DrTextureArgs a,
     }
   }
   __syncthreads();
-  const int C = a.channels, per = C / N;  // elements per pixel
+  constexpr int N = 4;
+  const int C = a.channels, per = (C + N - 1) / N;  // elements per pixel
   const int count = (int)min((int64_t)256, pixels - pixel0);
   // A step of 256 elements moves (pixel, element) by (dj, de).
   const int dj = 256 / per, de = 256 % per;
   int j = (int)threadIdx.x / per, e = (int)threadIdx.x % per;
   for (; j < count;) {
     const WideLookup<CUBE>& W = s_lookup[j];
-    const float* texels = a.texels + (int64_t)W.image * a.num_texels * C + e * N;
+    const int at = min(e * N, C - N);
+    const float* texels = a.texels + (int64_t)W.image * a.num_texels * C + at;
     auto fetch = [&](uint32_t index, float(&v)[N]) {
       if (index != kNoTexel) {
         load_floats(texels + (size_t)index * C, v);
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(256) void tex_fwd_wide_kernel(DrTextureArgs a,
         for (int c = 0; c < N; ++c) res[c] = res[c] * (1.0f - frac) + above[c] * frac;
       }
     }
-    store_floats(out + (pixel0 + j) * C + e * N, res);
+    store_floats(out + (pixel0 + j) * C + at, res);
     j += dj;
     e += de;
     if (e >= per) {
@@ -1099,12 +1103,8 @@ extern "C" int dr_texture_forward(const DrTextureArgs* a, float* out, void* stre
     const hipStream_t st = (hipStream_t)stream;
     if constexpr (NC > 0)
       tex_fwd_kernel<NC, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
-    else if (args.channels % 4 == 0)
-      tex_fwd_wide_kernel<4, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
-    else if (args.channels % 2 == 0)
-      tex_fwd_wide_kernel<2, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
     else
-      tex_fwd_wide_kernel<1, CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
+      tex_fwd_wide_kernel<CUBE, FILTER, BOUNDARY><<<blocks, 256, 0, st>>>(args, out);
     return launch_status();
   });
 }

@@ -316,13 +316,13 @@ def test_texture_gradients_where_pixels_share_texels(filter_mode, pattern):
     assert_grads_close(grads[:1], grads[1:])
 
 
-@pytest.mark.parametrize("channels", [5, 6, 8, 20, 300])
+@pytest.mark.parametrize("channels", [5, 6, 7, 8, 20, 300])
 @pytest.mark.parametrize("boundary", [*BOUNDARIES, "cube"])
 @pytest.mark.parametrize("tex_batch", [1, 2])
 def test_texture_many_channels(channels, boundary, tex_batch):
-    # More than four channels go one, two or four to a lane, 300 of them past a workgroup's
-    # lanes; lookups that read nothing (NaN coordinates and levels, a zero direction), cube
-    # edges and corners, every filter; 2 x 20 x 24 pixels end in a partial workgroup.
+    # More than four channels go four to a lane, 300 of them past a workgroup's lanes; lookups
+    # that read nothing (NaN coordinates and levels, a zero direction), cube edges and corners,
+    # every filter; 2 x 20 x 24 pixels end in a partial workgroup.
     gen = torch.Generator().manual_seed(channels)
     cube = boundary == "cube"
     tex = torch.randn(tex_batch, *((6, 16, 16) if cube else (13, 18)), channels, generator=gen)
@@ -352,6 +352,30 @@ def test_texture_many_channels(channels, boundary, tex_batch):
         for ours, ref in zip(grads[1:], e_grads[1:]):
             if ours is not None:
                 assert_grads_close([ours[1:] if cube else ours], [ref[1:] if cube else ref])
+
+
+def test_texture_of_seven_channels_takes_no_longer_than_of_eight():
+    # Twice as long while counts that four does not divide went one channel to a lane.
+    h, w = 2160, 3840
+    grid = torch.stack(torch.meshgrid(torch.arange(h) / h, torch.arange(w) / w, indexing="ij"), -1)
+    uv = grid.flip(-1)[None].cuda().contiguous()
+    uv_da = torch.full((1, h, w, 4), 1.5 / 512, device="cuda")
+
+    def time(channels):
+        tex = torch.rand(1, 512, 512, channels, device="cuda")
+        mip = dr.texture_construct_mip(tex)
+        times = []
+        for _ in range(4):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                dr.texture(tex, uv, uv_da, mip=mip, filter_mode="linear-mipmap-linear")
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    assert time(7) < 1.4 * time(8)
 
 
 @pytest.mark.parametrize("channels", [1, 3, 4, 6])

@@ -244,9 +244,13 @@ __global__ __launch_bounds__(256) void interp_fwd_wide_kernel(DrInterpolateArgs 
 }
 
 // DIFF: num_diff > 0 (grad_db is written, grad_da read if given); without it the kernel holds
-// no derivative state. A tile that shows nothing only writes zeros (a barrier more where it
-// does: backward of 4 channels over 1.31 M triangles at 8 x 1024^2, 30 % of it covered, 156 ->
-// 149 us; of 32 channels over 82 k at 4 x 512^2 forward and backward 152 -> 140).
+// no derivative state. A tile that shows nothing only writes zeros, at the price of a barrier in
+// the others. Without and with that exit, us: 4 channels over 1.31 M triangles at 8 x 1024^2, 30 %
+// of it covered, 156 / 149, with derivatives 249 / 262; a small grid on eight 1024^2 images 104 / 74,
+// 8 channels with derivatives 195 / 163; a knot on 4 x 700 x 900, 4 channels with derivatives
+// 42 / 39; 16 channels over 82 k triangles at 4 x 512^2 58 / 55. (Leaving a pass at the table's own
+// barrier where nothing is to be added: 241 instead of 235 for 8 channels at 8 x 1024^2, 85 instead
+// of 74 for the small grid.)
 template <int NC, bool DIFF>
 __global__ __launch_bounds__(256) void interp_bwd_kernel(DrInterpolateArgs a,
                                                          const float* __restrict__ grad_out,

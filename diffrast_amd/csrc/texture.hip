@@ -744,7 +744,7 @@ __global__ __launch_bounds__(kMipTailThreads) void mip_up_tail(float* grad, int 
 constexpr int kMipStageLevels = 5;
 
 // The stages work on elements of a texel: float4 when the channels come in fours on a 16-byte
-// aligned buffer, else single channels. Consecutive lanes take a texel's elements in turn, so
+// aligned buffer, Rgb for three channels, else single channels. Consecutive lanes take a texel's elements in turn, so
 // that a wave's loads cover whole lines whatever the channel count (one lane per texel and
 // group of four, a pass per group, at 1024^2 x 16: 199 us to build the chain and 178 to fold
 // it; now 37 and 44).
@@ -763,10 +763,24 @@ __device__ __forceinline__ float4 add_quarter(float4 own, float4 parent) {
                      add_quarter(own.z, parent.z), add_quarter(own.w, parent.w));
 }
 
+// Three channels in one access, with no alignment but a float's (as three elements, the adjoint at
+// 1024^2 took 26 us; this way 21).
+struct Rgb {
+  float x, y, z;
+};
+__device__ __forceinline__ Rgb quad_mean(Rgb a, Rgb b, Rgb c, Rgb d) {
+  return {quad_mean(a.x, b.x, c.x, d.x), quad_mean(a.y, b.y, c.y, d.y),
+          quad_mean(a.z, b.z, c.z, d.z)};
+}
+__device__ __forceinline__ Rgb add_quarter(Rgb own, Rgb parent) {
+  return {add_quarter(own.x, parent.x), add_quarter(own.y, parent.y),
+          add_quarter(own.z, parent.z)};
+}
+
 // Elements of a texel that a stage takes at a time (LDS: 20 KB), and the LDS of the levels of a
 // tile 2^j texels across: even j in one buffer (at most 16 x 16), odd j in the other (8 x 8).
 template <class V>
-constexpr int kStageElements = 64 / (int)sizeof(V);
+constexpr int kStageElements = std::is_same_v<V, Rgb> ? 1 : 64 / (int)sizeof(V);
 template <class V>
 struct MipStage {
   V even[256 * kStageElements<V>], odd[64 * kStageElements<V>];
@@ -940,7 +954,7 @@ void stage_elements(int C, const void* texels, const void* base, F f) {
   switch (C) {
     case 1: return f(float(), integral_constant<int, 1>());
     case 2: return f(float(), integral_constant<int, 2>());
-    case 3: return f(float(), integral_constant<int, 3>());
+    case 3: return f(Rgb(), integral_constant<int, 1>());
     default: return f(float(), integral_constant<int, 0>());
   }
 }

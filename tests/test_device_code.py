@@ -21,6 +21,15 @@ def kernels(source, name):
     return {symbol: body for symbol, body in found if re.search(name, symbol)}
 
 
+def test_mip_stages_take_three_channels_in_one_access():
+    bodies = kernels("texture.hip", r"mip_(down|up)_stageI.*3RgbELi1E")
+    assert len(bodies) == 2
+    for symbol, body in bodies.items():
+        for access in ("load", "store"):
+            assert re.search(rf"global_{access}_dwordx3\b", body), symbol
+            assert not re.search(rf"global_{access}_dword(x2)?\b", body), symbol
+
+
 def test_antialias_reads_groups_of_four_channels_in_one_access():
     # More than four channels go in fours, 16 bytes an access (a path for fewer channels beside it
     # made the compiler split them into 12 and 4 bytes: a third slower at 8 channels).

@@ -530,6 +530,7 @@ def test_mip_chain_tile_stages(shape):
 @pytest.mark.parametrize("shape,offset", [
     ((1, 64, 64, 16), 0), ((2, 64, 32, 20), 0),  # whole passes of channels, and a partial one
     ((1, 64, 64, 8), 1),                         # the same on a buffer that is not aligned
+    ((2, 64, 96, 3), 0), ((1, 6, 32, 32, 3), 1),  # three channels in one access
     ((1, 96, 96, 5), 0), ((2, 32, 32, 17), 0),   # channels that do not come in fours
     ((3, 45, 30, 2), 0), ((1, 6, 24, 24, 3), 0),  # chains ending in one workgroup's levels
     ((1, 130, 70, 7), 0),                        # levels of their own before those

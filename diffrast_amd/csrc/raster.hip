@@ -150,9 +150,8 @@ uint32_t large_tiles_limit(const DrRasterGeometry& g, int64_t tiles) {
 
 // Places in the list of large triangles: one each for the triangles of a smaller mesh; a larger
 // one, whose records are the bulk of the workspace, has as many as it has tile lists. Triangles
-// beyond them are binned tile by tile in their own threads, one thread's walk for each 256
-// triangles' workgroup: 8000 triangles of 300 pixels on 1024^2 against 4097 places took 4.20 ms
-// to rasterize; with a place for each 0.80.
+// beyond them are binned tile by tile in their own threads: 8000 triangles of 300 pixels on 1024^2
+// against 4097 places took 4.20 ms to rasterize; with a place for each 0.80.
 constexpr int64_t kLargePlacesBelow = (int64_t)1 << 18;  // triangle instances
 uint32_t large_list_places(const DrRasterGeometry& g, int64_t lists) {
   const int64_t places =
